@@ -1405,7 +1405,7 @@ static int lowbit_host(int kind, bool mopa, size_t m, const smg_weights *w, uint
                      [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
                          const hipError_t e = mopa ? launch_gemm(d, m, dd, 1, (long)n, dl, 1, (long)k, 1.0f, p.fused,
                                                                  false, s)
-                                                   : launch_lowbit_gemv(d, m, dd, dl, p.fused, sc, s);
+                                                   : launch_lowbit_gemv(d, m, dd, dl, p.fused, sc, scratch, s);
                          return e == hipSuccess ? plan_tail(p, dd, 1, (long)n, m, n, false, s) : e;
                      });
 }
@@ -1681,7 +1681,7 @@ int smg_lowbit_matmul_dev(size_t m, const smg_weights *w, uint16_t *dst, const u
         scratch = dev_pool().get(w->device, stream, sb);
         if (!scratch) return fail(SMG_ENOMEM, "smg_lowbit_matmul_dev: scratch hipMalloc");
     }
-    hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, scratch, (hipStream_t)stream);
+    hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, scratch, sb, (hipStream_t)stream);
     if (e == hipSuccess) e = plan_tail(ep_p, dst, 1, (long)w->d.n, m, w->d.n, false, (hipStream_t)stream);
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_lowbit_matmul_dev", e);
 }
@@ -1700,13 +1700,13 @@ int smg_lowbit_matmul_dev_noalloc(size_t m, const smg_weights *w, uint16_t *dst,
     if (rc) return rc;
     if ((rc = check_dev_ptrs("smg_lowbit_matmul_dev_noalloc", w->device, stream, ep_p, {dst, lhs}))) return rc;
     const EpArgs &ea = ep_p.fused;
-    const size_t sb = lowbit_scratch_bytes(w->d, m, &ea);
+    const size_t sb = lowbit_scratch_bytes(w->d, m, &ea, SMG_NOALLOC_SCRATCH_BYTES);
     if (sb > SMG_NOALLOC_SCRATCH_BYTES)
         return fail(SMG_EINVAL, "smg_lowbit_matmul_dev_noalloc: the call needs more scratch than "
                                 "SMG_NOALLOC_SCRATCH_BYTES (fewer rows or a shorter K)");
     void *p = nullptr;
     if (sb && (rc = noalloc_scratch(w->device, &p))) return rc;
-    hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, p, (hipStream_t)stream);
+    hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, p, sb, (hipStream_t)stream);
     if (e == hipSuccess) e = plan_tail(ep_p, dst, 1, (long)w->d.n, m, w->d.n, false, (hipStream_t)stream);
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_lowbit_matmul_dev_noalloc", e);
 }

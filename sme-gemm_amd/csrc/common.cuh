@@ -755,4 +755,30 @@ __device__ __forceinline__ uint4 q4_deq8_bf16(uint32_t q, uint32_t s1, float mf,
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
+// ---- low-bit activations -----------------------------------------------------
+
+// Four f16 activations (two dwords) quantized with the block's inv and packed
+// into four int8 bytes: f32(a) * inv with one rounding (v_fma_mix_f32: the f16
+// operand widened exactly, a -0 addend leaves the product as it is), ties to
+// even (v_rndne_f32), then v_cvt_i32_f32, whose NaN gives 0 as the reference's
+// quantize_row does. No clamp is needed: |a| <= amax, inv <= 127/amax * (1 +
+// 2^-24), so |a * inv| rounds to at most 127 (and inv = 0 when amax is 0, inf
+// or NaN, leaving 0 or NaN).
+__device__ __forceinline__ uint32_t quant4(uint32_t w0, uint32_t w1, float inv) {
+    float f[4];
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(f[0]) : "v"(w0), "v"(inv), "v"(-0.0f));
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[1]) : "v"(w0), "v"(inv), "v"(-0.0f));
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(f[2]) : "v"(w1), "v"(inv), "v"(-0.0f));
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[3]) : "v"(w1), "v"(inv), "v"(-0.0f));
+    uint32_t q[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float r = __builtin_rintf(f[e]);
+        asm("v_cvt_i32_f32 %0, %1" : "=v"(q[e]) : "v"(r));
+    }
+    const uint32_t lo = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u);  // {q0, q1, 0, 0} (low bytes)
+    const uint32_t hi = __builtin_amdgcn_perm(q[3], q[2], 0x0c0c0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
 }  // namespace smg

@@ -30,6 +30,7 @@
 #include <atomic>
 
 #include "kernels.h"
+#include "lds_dma.cuh"
 #include "tile_store.cuh"
 
 namespace smg {
@@ -73,39 +74,6 @@ struct RArgs {
     uint32_t nh;
 };
 
-// LDS DMA: each lane's 16 (4) bytes from sbase + voff land at M0 + 16 (4) *
-// lane; sbase is wave-uniform (scalar registers), voff the lane's 32-bit byte
-// offset, so a step's addresses cost no vector instructions. The instructions
-// are issued from inline asm so that the compiler neither tracks them nor adds
-// waits of its own (it cannot tell which stage a DMA fills); the kernel's
-// explicit vmcnt waits and barriers order them. The "memory" clobber keeps LDS
-// reads from moving across an issue; s_nop covers the M0 write hazard. lds is a
-// wave-uniform LDS byte address. (M0 has no other user in this kernel, so
-// clobbering it is safe.)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16(const void *sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase),
-                 "s"(lds)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void *sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase),
-                 "s"(lds)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-__device__ __forceinline__ uint32_t lds_addr(const void *p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p;
-}
-
-// s_waitcnt vmcnt(n) (gfx9 encoding; expcnt and lgkmcnt left unwaited).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // At most n (uniform) steps' DMA still in flight.
 __device__ __forceinline__ void wait_vm_steps(int n) {
     if (n >= 3)
@@ -116,16 +84,6 @@ __device__ __forceinline__ void wait_vm_steps(int n) {
         wait_vm<PS>();
     else
         wait_vm<0>();
-}
-
-// Workgroup barrier that orders LDS accesses without waiting on outstanding
-// DMA (a release fence would wait for all of it): the empty asm statements keep
-// the compiler from moving memory accesses across it; the caller first waits
-// for the DMA the next step reads.
-__device__ __forceinline__ void barrier_lds() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
 }
 
 // Per-lane DMA offsets that do not change from step to step. Thread t loads
@@ -179,12 +137,6 @@ __device__ __forceinline__ ReadOff read_offsets(int kk, int cw, int lane) {
     o.q = A_BYTES + (kk * 256 + cw * 64 + lr) * 16 + lg * 4;
     o.s = A_BYTES + B_BYTES + kk * 512 + (cw * 64 + lr) * 2;
     return o;
-}
-
-typedef const __attribute__((address_space(3))) uint8_t lds_u8_t;
-template <class T>
-__device__ __forceinline__ T lds_load(uint32_t addr) {
-    return *(const __attribute__((address_space(3))) T *)(lds_u8_t *)(uintptr_t)addr;
 }
 
 // Stage at LDS byte address sb: row tile i's fragment at o.a + 2048 i, column

@@ -64,9 +64,19 @@ hipError_t launch_q4_gemv_chained(const WDev &w, size_t m, uint16_t *dst, const 
 // rows outside the persistent kernel, or blocks too large to quantize
 // in-kernel). ep: the call's fused op-graph, which decides whether the
 // persistent kernel serves (then 0); null sizes for the other kernels.
-size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep = nullptr);
+// limit: the most scratch the caller can give; the many-row GEMM (lowbit_gemm)
+// serves a call only where its own scratch fits.
+size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep = nullptr, size_t limit = ~(size_t)0);
+// scratch_bytes: what lowbit_scratch_bytes returned for the call.
 hipError_t launch_lowbit_gemv(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs,
-                              const EpArgs &ep, void *scratch, hipStream_t s);
+                              const EpArgs &ep, void *scratch, size_t scratch_bytes, hipStream_t s);
+
+// The many-row form (lowbit_gemm.hip): from LOWBIT_GEMM_ROWS rows, blocks of
+// 64, 128 or 256. lowbit_gemm_bytes is its scratch, 0 where it does not serve.
+constexpr size_t LOWBIT_GEMM_ROWS = 9;
+size_t lowbit_gemm_bytes(const WDev &w, size_t m);
+hipError_t launch_lowbit_gemm(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs, const EpArgs &ep,
+                              void *scratch, hipStream_t s);
 
 // MFMA GEMM over any weight kind (Q4 / Q2 / Q1 dequantized to f16/bf16 in LDS,
 // or dense), C[i,j] at dst[i*rs + j*cs] = ep(to16(beta * acc)).

@@ -290,30 +290,6 @@ __device__ __forceinline__ int32_t group_sum_i32(int32_t a, uint32_t gl) {
     return a;
 }
 
-// Four f16 activations (two dwords) quantized with the block's inv and packed
-// into four int8 bytes: f32(a) * inv with one rounding (v_fma_mix_f32: the f16
-// operand widened exactly, a -0 addend leaves the product as it is), ties to
-// even (v_rndne_f32), then v_cvt_i32_f32, whose NaN gives 0 as the reference's
-// quantize_row does. No clamp is needed: |a| <= amax, inv <= 127/amax * (1 +
-// 2^-24), so |a * inv| rounds to at most 127 (and inv = 0 when amax is 0, inf
-// or NaN, leaving 0 or NaN).
-__device__ __forceinline__ uint32_t quant4(uint32_t w0, uint32_t w1, float inv) {
-    float f[4];
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(f[0]) : "v"(w0), "v"(inv), "v"(-0.0f));
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[1]) : "v"(w0), "v"(inv), "v"(-0.0f));
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(f[2]) : "v"(w1), "v"(inv), "v"(-0.0f));
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(f[3]) : "v"(w1), "v"(inv), "v"(-0.0f));
-    uint32_t q[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float r = __builtin_rintf(f[e]);
-        asm("v_cvt_i32_f32 %0, %1" : "=v"(q[e]) : "v"(r));
-    }
-    const uint32_t lo = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u);  // {q0, q1, 0, 0} (low bytes)
-    const uint32_t hi = __builtin_amdgcn_perm(q[3], q[2], 0x0c0c0400u);
-    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-}
-
 // LDS: q [MR][kq + 16] i8, for one row later the fold's y and x, each [16
 //      CG][nbq + 4] f32 (the products have read q by then) | s [MR][nbq] f32 |
 //      -sum(q) [MR][nbq] i32 | block sums [MR][16 CG][nbq + 4] i32 (one row:
@@ -1570,7 +1546,9 @@ size_t prequant_bytes(size_t m, size_t kq, size_t nbq) { return (m * kq + 255) /
 
 }  // namespace
 
-size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep) {
+size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep, size_t limit) {
+    const size_t gb = lowbit_gemm_bytes(w, m);
+    if (gb && gb <= limit) return gb;
     const TileGeo sg = tile_geometry(w, m);
     if (sg.ok && ep && row_shape(w, m, sg, *ep).tpw > 0) return 0;  // lowbit_row quantizes in-kernel
     if (sg.ok) return m > 1 ? prequant_bytes(m, sg.kq, sg.nbq) : 0;
@@ -1579,7 +1557,9 @@ size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep) {
 }
 
 hipError_t launch_lowbit_gemv(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs,
-                              const EpArgs &ep, void *scratch, hipStream_t s) {
+                              const EpArgs &ep, void *scratch, size_t scratch_bytes, hipStream_t s) {
+    const size_t gb = lowbit_gemm_bytes(w, m);
+    if (gb && gb <= scratch_bytes) return launch_lowbit_gemm(w, m, dst, lhs, ep, scratch, s);
     const TileGeo sg = tile_geometry(w, m);
     if (sg.ok) {
         const size_t cb = cell_grid_rows(w.nchunks) * w.n_pad * 64;

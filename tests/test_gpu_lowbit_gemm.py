@@ -1,0 +1,118 @@
+"""The many-row 2-bit / 1-bit int8 GEMM (lowbit_gemm) against the oracle, bit
+for bit: quantization, block sums, the in-order fold and the op-graph are the
+same steps as the decode kernels', so every output is identical."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (m, n, k): the fewest rows served, 16-row tile edges, 32- and 64-row tile
+# edges, ragged N (one 128-column tile and several) and K below, at and past a
+# 256-depth step and a Q1 group (512), K not a multiple of 8 (the element-wise
+# row loads) and several steps with a last partial block
+SHAPES = [(9, 128, 256), (16, 5, 64), (17, 130, 300), (31, 257, 512), (32, 384, 1024), (33, 1000, 777),
+          (63, 128, 4096), (64, 129, 520), (65, 640, 2049), (130, 300, 1288),
+          # 32-row, 64-row and 64 x 128 tiles (more 16-row tiles than the
+          # device takes at once), ragged rows and columns
+          (130, 8200, 300), (300, 9001, 256), (400, 16300, 328)]
+BOOKS = [(-1, 0, 1, 0), (-2, -1, 1, 2), (-128, 127, 3, -7)]
+
+
+def _inputs(orc, rng, m, n, k, block, bits):
+    nbk = -(-k // block)
+    scales = orc.f32_to_f16(rng.uniform(-0.05, 0.05, n * nbk).astype(np.float32))
+    a = orc.f32_to_f16(rng.standard_normal(m * k).astype(np.float32))
+    codes = rng.integers(0, 256, (k * n * bits + 7) // 8, dtype=np.uint8)
+    return a, codes, scales
+
+
+def _both(smg, orc, a, codes2, signs, scales, m, n, k, block, book, ep=None, nodes=(), act=None):
+    q2 = smg.Q2Weights(codes2, scales, n, k, smg.Q2Params(block).with_codebook(book))
+    got = np.full(m * n, 0x4880, np.uint16)
+    smg.matmul_q2_ep(a, q2, got, m, ep or smg.Epilogue())
+    want = orc.matmul_lowbit_ep(2, a, codes2, scales, m, n, k, block, nodes, act, codebook=book)
+    assert np.array_equal(got, want), "q2"
+    for layout in (smg.WeightLayout.OutIn, smg.WeightLayout.InOut):
+        q1 = smg.Q1Weights(signs, scales, layout, n, k, block)
+        got = np.full(m * n, 0x4880, np.uint16)
+        smg.matmul_q1_ep(a, q1, got, m, ep or smg.Epilogue())
+        want = orc.matmul_lowbit_ep(1, a, signs, scales, m, n, k, block, nodes, act,
+                                    inout=layout == smg.WeightLayout.InOut)
+        assert np.array_equal(got, want), f"q1 layout {layout}"
+
+
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("si", range(len(SHAPES)))
+def test_many_rows_match_reference_bits(smg, orc, si, block):
+    m, n, k = SHAPES[si]
+    rng = np.random.default_rng(1000 * block + si)
+    a, codes2, scales = _inputs(orc, rng, m, n, k, block, 2)
+    signs = rng.integers(0, 256, (k * n + 7) // 8, dtype=np.uint8)
+    _both(smg, orc, a, codes2, signs, scales, m, n, k, block, BOOKS[si % 3])
+
+
+@pytest.mark.parametrize("graph", ["bias", "bias_silu", "scale_bias_gelu", "interpreted"])
+def test_many_rows_epilogue_bits(smg, orc, graph):
+    """Each compiled store and the interpreted one, over ragged edges."""
+    m, n, k, block = 70, 203, 640, 128
+    rng = np.random.default_rng(77)
+    a, codes2, scales = _inputs(orc, rng, m, n, k, block, 2)
+    signs = rng.integers(0, 256, (k * n + 7) // 8, dtype=np.uint8)
+    b = orc.f32_to_f16(rng.uniform(-4, 4, n).astype(np.float32))
+    s = orc.f32_to_f16(rng.uniform(0.5, 1.5, n).astype(np.float32))
+    r = orc.f32_to_f16(rng.uniform(0.5, 1.5, m).astype(np.float32))
+    t = orc.f32_to_f16(rng.uniform(-1, 1, m * n).astype(np.float32))
+    ep, nodes, act = {
+        "bias": (smg.Epilogue().add_col(b), [(4, 0, 0.0, b, 0)], None),
+        "bias_silu": (smg.Epilogue().add_col(b).silu(), [(4, 0, 0.0, b, 0)], 3),
+        "scale_bias_gelu": (smg.Epilogue().mul_col(s).add_col(b).gelu(),
+                            [(5, 0, 0.0, s, 0), (4, 0, 0.0, b, 0)], 2),
+        "interpreted": (smg.Epilogue().mul_row(r).add_tensor(t).sigmoid(),
+                        [(3, 0, 0.0, r, 0), (6, 0, 0.0, t, n)], 5),
+    }[graph]
+    _both(smg, orc, a, codes2, signs, scales, m, n, k, block, (-1, 0, 1, 0), ep, nodes, act)
+
+
+def test_many_rows_special_activations(smg, orc):
+    """Blocks of zeros, infinities, NaN and the smallest subnormals, and rows
+    that differ only in one block: amax, inv and s as quantize_row gives them
+    (NaN outputs compared as NaN: their bits are the platform's)."""
+    m, n, k, block = 40, 130, 512, 128
+    rng = np.random.default_rng(5)
+    a, codes2, scales = _inputs(orc, rng, m, n, k, block, 2)
+    av = a.reshape(m, k)
+    av[1, :128] = 0
+    av[2, 130] = 0x7C00
+    av[3, 260] = 0x7E00
+    av[4, 384:] = 1
+    av[5, :] = 0x7BFF
+    av[17, 0] = 0xFC00
+    av[33, 511] = 0xFE01
+    q2 = smg.Q2Weights(codes2, scales, n, k, smg.Q2Params(block))
+    got = np.zeros(m * n, np.uint16)
+    smg.matmul_q2(a, q2, got, m)
+    want = orc.lowbit_reference(2, a, codes2, scales, m, n, k, block)
+    nan = lambda x: (x & 0x7FFF) > 0x7C00  # noqa: E731
+    assert np.array_equal(nan(got), nan(want))
+    assert np.array_equal(got[~nan(want)], want[~nan(want)])
+
+
+def test_noalloc_keeps_the_calls_it_took(smg, orc):
+    """961 rows at K = 4096: the GEMM's scratch (16-row tiles) would pass the
+    static array, the GEMV's fits it -- the call runs there, the same bits."""
+    import torch
+    m, n, k, block = 961, 128, 4096, 128
+    rng = np.random.default_rng(9)
+    a, codes2, scales = _inputs(orc, rng, m, n, k, block, 2)
+    w = smg.Q2Weights(codes2, scales, n, k, smg.Q2Params(block))
+    ad = torch.from_numpy(a.view(np.int16)).cuda()
+    out = [torch.zeros(m * n, dtype=torch.int16, device="cuda") for _ in range(2)]
+    fn = smg.lib().smg_lowbit_matmul_dev_noalloc
+    fn.argtypes = [C.c_size_t] + [C.c_void_p] * 5
+    st = torch.cuda.current_stream().cuda_stream
+    assert fn(m, w._h, out[0].data_ptr(), ad.data_ptr(), None, st) == 0
+    smg.matmul_q2(ad, w, out[1], m)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1])
