@@ -1501,6 +1501,18 @@ static size_t footprint(size_t rows, long rs, size_t cols, long cs) {
     return rows && cols ? (rows - 1) * (size_t)rs + (cols - 1) * (size_t)cs + 1 : 0;
 }
 
+// The strided product as a dense GEMM that reads B where it is: a column-major
+// B is already K-contiguous. (Packing reads all of B before C is written, so a
+// B that shares memory with C keeps it.)
+static bool strided_direct(DenseGemm *d, size_t m, size_t n, size_t k, uint16_t *dst, long dst_cs, long dst_rs,
+                           int read_dst, const uint16_t *lhs, long lhs_cs, long lhs_rs, const uint16_t *rhs,
+                           long rhs_cs, long rhs_rs, float alpha, float beta) {
+    *d = {lhs, rhs, dst, m, n, k, n, lhs_rs, rhs_cs, dst_rs, dst_cs, beta, alpha, read_dst != 0};
+    if (lhs_cs != 1 || rhs_rs != 1 || !gemm_dense_supported(*d)) return false;
+    const uint16_t *rend = rhs + footprint(k, rhs_rs, n, rhs_cs), *dend = dst + footprint(m, dst_rs, n, dst_cs);
+    return rend <= dst || dend <= rhs;
+}
+
 static int run_host(bool bf16, const char *name, size_t m, size_t n, size_t k, uint16_t *dst, long dst_cs,
                     long dst_rs, int read_dst, const uint16_t *lhs, long lhs_cs, long lhs_rs,
                     const uint16_t *rhs, long rhs_cs, long rhs_rs, uint16_t alpha_bits, uint16_t beta_bits) {
@@ -1532,6 +1544,10 @@ static int run_host(bool bf16, const char *name, size_t m, size_t n, size_t k, u
                              const hipError_t e = hipMemcpyAsync(raw, rhs, rhs_elems * 2, hipMemcpyHostToDevice, s);
                              if (e != hipSuccess) return e;
                          }
+                         DenseGemm dg;
+                         if (strided_direct(&dg, m, n, k, dd, dst_cs, dst_rs, read_dst, dl, lhs_cs, lhs_rs, raw, rhs_cs,
+                                            rhs_rs, alpha, beta))
+                             return launch_gemm_dense(dg, ea, bf16, s);
                          hipError_t e = launch_pack_dense_strided(raw, rhs_rs, rhs_cs, n, k, d.n_pad, d.k_pad,
                                                                   dense, s);
                          if (e != hipSuccess) return e;
@@ -1580,6 +1596,13 @@ int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long
     int rc = check_dev_ptrs("smg_gemm_run_dev", device, stream, EpPlan{},
                             {dst, k ? lhs : nullptr, k ? rhs : nullptr});
     if (rc) return rc;
+    const float alpha = half_bits_to_float(alpha_bits, bf16 != 0), beta = half_bits_to_float(beta_bits, bf16 != 0);
+    DenseGemm dg;
+    if (strided_direct(&dg, m, n, k, dst, dst_cs, dst_rs, read_dst, lhs, lhs_cs, lhs_rs, rhs, rhs_cs, rhs_rs, alpha,
+                       beta)) {
+        const hipError_t e = launch_gemm_dense(dg, EpArgs{}, bf16 != 0, (hipStream_t)stream);
+        return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_gemm_run_dev", e);
+    }
     WDev d = {};
     d.kind = bf16 ? W_BF16 : W_F16;
     d.n = n;
@@ -1594,8 +1617,8 @@ int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long
         d.dense = dense;
         EpArgs ea = {};
         const bool b = bf16 != 0;
-        e = launch_gemm(d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, half_bits_to_float(beta_bits, b), ea, b,
-                        (hipStream_t)stream, read_dst != 0, half_bits_to_float(alpha_bits, b));
+        e = launch_gemm(d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ea, b, (hipStream_t)stream,
+                        read_dst != 0, alpha);
     }
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_gemm_run_dev", e);
 }

@@ -94,6 +94,21 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
 hipError_t launch_pack_dense_strided(const uint16_t *rhs, long rhs_rs, long rhs_cs, size_t n, size_t k,
                                      size_t n_pad, size_t k_pad, uint16_t *dense, hipStream_t s);
 
+// The dense GEMM over K-contiguous operands (gemm_dense.hip): A [m][lda], B
+// [n][ldb] (brows >= n rows can be read), C[i,j] at dst[i*dst_rs + j*dst_cs].
+// read_dst: with no graph alpha * C + beta * A@B with one rounding, with one
+// alpha * C added after it.
+struct DenseGemm {
+    const uint16_t *a, *b;
+    uint16_t *dst;
+    size_t m, n, k, brows;
+    long lda, ldb, dst_rs, dst_cs;
+    float beta, alpha;
+    bool read_dst;
+};
+bool gemm_dense_supported(const DenseGemm &d);
+hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hipStream_t s);
+
 // Q4 GEMM with register-resident weights (gemm_q4r.hip): f16 or bf16
 // activations, block >= 32, K a multiple of 64, row-major 16-byte-aligned A.
 // launch_gemm uses it whenever q4r_supported holds.

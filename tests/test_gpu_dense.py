@@ -1,0 +1,116 @@
+"""The DMA-staged dense GEMM (gemm_dense): every tile of its rule, K tails,
+strided operands and stores, against a float64 product of the same 16-bit
+inputs. The result is rounded to 16 bits once from an f32 sum, so the bound is
+half an ulp of the result plus the f32 sum's error (K products, each within
+2^-24 of the running sum's magnitude), stated relative to 1 + |w|."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# one shape a tile: 256x256, 128x256, 64x128, 64x64, 32x64, ragged in m and n
+TILES = [(4000, 4090, 520), (500, 14300, 2056), (1000, 3001, 520), (250, 4001, 520), (61, 499, 520)]
+# K edges on the smallest tile: one step, one chunk past it, one chunk short of
+# two, whole steps
+KS = [(33, 130, 64), (33, 130, 72), (33, 130, 120), (33, 130, 128), (5, 7, 1000)]
+
+
+def _tol(k, bf16):
+    return (2.0 ** -8 if bf16 else 2.0 ** -11) + k * 2.0 ** -24
+
+
+def _mats(m, n, k, bf16, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    t = torch.bfloat16 if bf16 else torch.float16
+    a = torch.randn(m, k, generator=g, device="cuda").to(t)
+    b = (torch.randn(k, n, generator=g, device="cuda") / k ** 0.5).to(t)
+    return a, b
+
+
+def _bits(x):
+    import torch
+    return x.contiguous().cpu().view(torch.int16).numpy().view(np.uint16)
+
+
+def _check(got, want, k, bf16):
+    import torch
+    err = ((got.double() - want).abs() / (1 + want.abs())).max().item()
+    assert err <= _tol(k, bf16), err
+    assert bool(torch.isfinite(got).all())
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("m,n,k", TILES + KS)
+def test_packed_product(smg, m, n, k, bf16):
+    import torch
+    a, b = _mats(m, n, k, bf16, m + n + k)
+    p = (smg.prepack_bf16 if bf16 else smg.prepack_f16)(_bits(b), n, k)
+    c = torch.empty(m, n, dtype=a.dtype, device="cuda")
+    (smg.matmul_bf16_packed if bf16 else smg.matmul_f16_packed)(a, p, c, m)
+    _check(c, a.double() @ b.double(), k, bf16)
+
+
+@pytest.mark.parametrize("graph", ["bias", "scale_bias_relu", "interpreted"])
+@pytest.mark.parametrize("m,n,k", TILES)
+def test_packed_epilogue(smg, m, n, k, graph):
+    """The compiled stores and the interpreted one on each tile (row-major and,
+    interpreted, column-major C). beta 0.5 is exact in the store."""
+    import torch
+    a, b = _mats(m, n, k, False, 3)
+    p = smg.prepack_f16(_bits(b), n, k)
+    bias, scale = (torch.randn(n, device="cuda").half() for _ in range(2))
+    row = torch.randn(m, device="cuda").half()
+    h = (0.5 * (a.double() @ b.double())).half().double()  # the graph runs on the rounded product
+    g = smg.Gemm(a, p, m).beta(0.5)
+    c = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    if graph == "bias":
+        g, want = g.add_col(bias), h + bias.double()
+    elif graph == "scale_bias_relu":
+        g, want = g.mul_col(scale).add_col(bias).relu(), (h * scale.double() + bias.double()).clamp(min=0)
+    else:
+        g, want = g.col_major_output().mul_row(row).add_col(bias), h * row.double()[:, None] + bias.double()
+        c = torch.empty(n, m, dtype=torch.float16, device="cuda")
+    g.run(c)
+    got = c.t() if graph == "interpreted" else c
+    # the product's rounding may fall to either side (one f16 ulp, scaled by
+    # the largest |factor| drawn, below 5), then the store's own half ulp
+    err = ((got.double() - want).abs() / (1 + want.abs() + 5 * h.abs())).max().item()
+    assert err <= 2 * _tol(k, False), err
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.75])
+@pytest.mark.parametrize("bcol", [True, False])
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("m,n,k", TILES[2:] + KS)
+def test_strided_views(smg, m, n, k, bf16, bcol, alpha):
+    """Views of larger arrays whose other elements are NaN (nothing outside a
+    view is read into a sum), C a padded view; a column-major B is read in
+    place, a row-major one packed."""
+    import torch
+    a, b = _mats(m, n, k, bf16, 7)
+    lda, ldb, ldc = k + 8, (k if bcol else n) + 16, n + 3
+    nan = lambda r, c: torch.full((r, c), float("nan"), dtype=a.dtype, device="cuda")  # noqa: E731
+    av, bv, cv = nan(m, lda), nan(n if bcol else k, ldb), nan(m, ldc)
+    av[:, :k] = a
+    bv[:, :k if bcol else n] = b.t() if bcol else b
+    c0 = torch.randn(m, n, device="cuda").to(a.dtype)
+    if alpha:
+        cv[:, :n] = c0
+    f = smg.gemm_bf16 if bf16 else smg.gemm_f16
+    f(m, n, k, cv, ldc, 1, av, lda, 1, bv, *((1, ldb) if bcol else (ldb, 1)), alpha, 1.0)
+    want = a.double() @ b.double() + alpha * c0.double()
+    _check(cv[:, :n], want, k, bf16)
+    assert bool(cv[:, n:].isnan().all())  # the padding is untouched
+
+
+def test_strided_result_may_share_memory_with_b(smg):
+    """C over B's own memory (packing reads all of B first): the direct read
+    stays off it."""
+    import torch
+    m = n = k = 256
+    a, b = _mats(m, n, k, False, 11)
+    bt = b.t().contiguous()
+    want = a.double() @ b.double()
+    smg.gemm_f16(m, n, k, bt, n, 1, a, k, 1, bt, 1, k, 0.0, 1.0)
+    _check(bt, want, k, False)
