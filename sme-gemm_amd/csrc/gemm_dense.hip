@@ -25,7 +25,7 @@
 // reads: the DMA is never drained inside the loop. (128 x 256, a wave 64 x 64,
 // where 256-row tiles leave compute units idle.)
 // gemm_dense_tile: smaller tiles of four waves for smaller products.
-// What bounds them: 8192^3 runs at 1.36 PF/s, 1.58 us a step of 64 depths where
+// What bounds them: 8192^3 runs at 1.42 PF/s, 1.5 us a step of 64 depths where
 // the products alone are 0.85 us at the nominal clock; the fragment reads and
 // the refill take the LDS about as long as the products take the matrix cores,
 // and the slots' barriers keep the two from overlapping fully.
@@ -56,17 +56,13 @@ struct DArgs {
     float act_alpha;
 };
 
-// Chunks of a row past K read these zeros.
-__device__ const uint4 dense_zeros[1] = {{0, 0, 0, 0}};
-
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// dma16 with a 64-bit address per lane
-__device__ __forceinline__ void dma16_lane(const void *p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds)
-                 : "memory", "m0");
+// The operands as buffer resources from the tile's first row on: rows past the
+// last read zeros (never stored), and so do the last step's chunks past K,
+// whose lanes take the offset OOB.
+__device__ __forceinline__ rsrc4_t dense_rsrc(const uint16_t *p, uint32_t row0, uint32_t rows, long ld, uint32_t k) {
+    const uint64_t bytes = ((uint64_t)(rows - 1 - row0) * ld + k) * 2;
+    return make_rsrc4(p + (size_t)row0 * ld, (uint32_t)(bytes < OOB ? bytes : OOB));
 }
-#pragma clang diagnostic pop
 
 template <bool BF16>
 __device__ __forceinline__ float4_t mfma16(const u32x4_t &a, const u32x4_t &b, float4_t c) {
@@ -176,7 +172,7 @@ template <int BM, bool BF16, int EPV>
 __global__ void __launch_bounds__(DB_NT) gemm_dense_big(DArgs g, EpArgs ep) {
     using T = DBig<BM>;
     constexpr int RT = T::RT, RH = 16 * RT;  // rows of a wave's row half
-    __shared__ __align__(16) uint8_t ring[2 * T::STAGE];
+    __shared__ __align__(1024) uint8_t ring[2 * T::STAGE];
     const int t = threadIdx.x, lane = t % 64, lr = lane % 16, lg = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(t / 64);
     const int wr = wave / 4, wc = wave % 4;
@@ -189,67 +185,49 @@ __global__ void __launch_bounds__(DB_NT) gemm_dense_big(DArgs g, EpArgs ep) {
     // DMA sources: instruction q of a half moves its chunks (8q + wave) * 64 +
     // lane: row p / 8 of the half, slot p % 8. Half h of the rows holds rows RH h
     // .. RH h + RH - 1 of each wave row's 2 RH, half h of the columns 32h .. 32h +
-    // 31 of each wave column's 64. Rows past the operands repeat the last one.
-    const uint8_t *const abase = (const uint8_t *)(g.a + (size_t)row0 * g.lda);
-    const uint8_t *const bbase = (const uint8_t *)(g.b + (size_t)col0 * g.ldb);
-    uint32_t ao[2][T::QA], bo[2][T::QB], chunk;
-    {
-        const uint32_t slot = lane % 8, r8 = lane / 8;
-        chunk = slot ^ r8;  // row % 8 is lane / 8 in every piece
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int q = 0; q < T::QA; q++) {
-                const uint32_t r = (q * 8 + wave) * 8 + r8;
-                const uint32_t ar = min((r / RH) * (2 * RH) + h * RH + r % RH, g.m - 1 - row0);
-                ao[h][q] = (uint32_t)(ar * g.lda * 2) + chunk * 16;
-            }
-#pragma unroll
-            for (int q = 0; q < T::QB; q++) {
-                const uint32_t r = (q * 8 + wave) * 8 + r8;
-                const uint32_t br = min((r / 32) * 64 + h * 32 + r % 32, g.brows - 1 - col0);
-                bo[h][q] = (uint32_t)(br * g.ldb * 2) + chunk * 16;
-            }
-        }
-    }
+    // 31 of each wave column's 64. An address is a scalar part (the
+    // instruction's rows and the step) and the lane's row and chunk.
+    const rsrc4_t ra = dense_rsrc(g.a, row0, g.m, g.lda, g.k), rb = dense_rsrc(g.b, col0, g.brows, g.ldb, g.k);
+    const uint32_t lda2 = (uint32_t)g.lda * 2, ldb2 = (uint32_t)g.ldb * 2;
+    const uint32_t chunk = (lane % 8) ^ (lane / 8);  // row % 8 is lane / 8 in every piece
+    const uint32_t va = (lane / 8) * lda2 + chunk * 16, vb = (lane / 8) * ldb2 + chunk * 16;
     // half h of the rows (columns) of a step into its stage
     auto dma = [&](uint32_t step, int h, auto cols_c) __attribute__((always_inline)) {
         constexpr bool COLS = decltype(cols_c)::value;
-        constexpr int Q = COLS ? T::QB : T::QA;
+        constexpr int Q = COLS ? T::QB : T::QA, WR = COLS ? 32 : RH;
         const uint32_t ks = min(step, last);
         const uint32_t dst = lds0 + (step & 1) * T::STAGE + (COLS ? 2 * T::AH + h * T::BH : h * T::AH) + wave * 1024;
-        const uint8_t *base = (COLS ? bbase : abase) + (size_t)ks * 128;
-        const uint32_t *o = COLS ? bo[h] : ao[h];
-        if (ks * 64 + 64 <= g.k) {
+        uint32_t v = COLS ? vb : va;
+        if (ks * 64 + 64 > g.k) v = ks * 64 + chunk * 8 < g.k ? v : OOB;
 #pragma unroll
-            for (int q = 0; q < Q; q++) dma16(base, o[q], dst + q * 8192);
-        } else {  // the last step's chunks past K are zeros
-            const bool in = ks * 64 + chunk * 8 < g.k;
-#pragma unroll
-            for (int q = 0; q < Q; q++)
-                dma16_lane(in ? (const void *)(base + o[q]) : (const void *)dense_zeros, dst + q * 8192);
+        for (int q = 0; q < Q; q++) {
+            const uint32_t r = (q * 8 + wave) * 8, row = (r / WR) * (2 * WR) + h * WR + r % WR;
+            dma16_buf(COLS ? rb : ra, v, row * (COLS ? ldb2 : lda2) + ks * 128, dst + q * 8192);
         }
     };
     constexpr std::integral_constant<bool, false> rows;
     constexpr std::integral_constant<bool, true> cols;
     // fragment of row (column) tile i of a half, depths 32 kk ..: this lane's 16
-    // bytes of row lr
-    const uint32_t f0 = (lg ^ (lr & 7)) << 4, f1 = ((4 + lg) ^ (lr & 7)) << 4;
-    const uint32_t fa = (wr * RH + lr) * 128, fb = (wc * 32 + lr) * 128;
+    // bytes of row lr. (The addresses are opaque, so that the tiles are constant
+    // offsets of one register instead of a register each.)
+    const uint32_t f0 = lr * 128 + ((lg ^ (lr & 7)) << 4);
+    const uint32_t fa = lds0 + wr * RH * 128 + f0, fb = lds0 + 2 * T::AH + wc * 32 * 128 + f0;
     auto read_a = [&](uint32_t step, int h, u32x4_t (&x)[RT][2]) __attribute__((always_inline)) {
-        const uint32_t b = lds0 + (step & 1) * T::STAGE + h * T::AH + fa;
+        uint32_t b0 = fa + (step & 1) * T::STAGE + h * T::AH, b1 = b0 ^ 64;
+        asm volatile("" : "+v"(b0), "+v"(b1));
 #pragma unroll
         for (int i = 0; i < RT; i++) {
-            x[i][0] = lds_load<u32x4_t>(b + f0 + i * 2048);
-            x[i][1] = lds_load<u32x4_t>(b + f1 + i * 2048);
+            x[i][0] = lds_load<u32x4_t>(b0 + i * 2048);
+            x[i][1] = lds_load<u32x4_t>(b1 + i * 2048);
         }
     };
     auto read_b = [&](uint32_t step, int h, u32x4_t (&x)[2][2]) __attribute__((always_inline)) {
-        const uint32_t b = lds0 + (step & 1) * T::STAGE + 2 * T::AH + h * T::BH + fb;
+        uint32_t b0 = fb + (step & 1) * T::STAGE + h * T::BH, b1 = b0 ^ 64;
+        asm volatile("" : "+v"(b0), "+v"(b1));
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            x[j][0] = lds_load<u32x4_t>(b + f0 + j * 2048);
-            x[j][1] = lds_load<u32x4_t>(b + f1 + j * 2048);
+            x[j][0] = lds_load<u32x4_t>(b0 + j * 2048);
+            x[j][1] = lds_load<u32x4_t>(b1 + j * 2048);
         }
     };
 
@@ -333,11 +311,16 @@ __global__ void __launch_bounds__(DB_NT) gemm_dense_big(DArgs g, EpArgs ep) {
     wait_vm<0>();  // the steps issued past the last
     __syncthreads();
 
+    // (the thread's place, opaque: the loop then keeps none of what derives from
+    // it for the store)
+    int to = t;
+    asm volatile("" : "+v"(to));
+    const int lro = to % 16, lgo = to % 64 / 16;
     // Store, a row half of every wave at a time: the first RH staged
     // rows from wave row 0, the rest from wave row 1.
     uint16_t *stg = (uint16_t *)ring;
     float *colv = (float *)(ring + T::STG), *rowv = colv + EP_FUSED * DB;
-    const int cl = (t % 32) * 8, rl = t / 32;
+    const int cl = (to % 32) * 8, rl = to / 32;
     EpCols cv;
     if constexpr (EPV == 0) ep_load_vectors<BF16, BM, DB, DB_NT>(g.st, ep, colv, rowv, row0, col0);
     if constexpr (EPV >= 2) ep_cols_load<EPV>(g.col_a, g.col_b, col0 + cl, g.n, cv);
@@ -355,7 +338,7 @@ __global__ void __launch_bounds__(DB_NT) gemm_dense_big(DArgs g, EpArgs ep) {
 #pragma unroll
                 for (int j = 0; j < 2; j++)
                     dense_stage4<BF16>(g, c[ch][i][j],
-                                       stg + (wr * RH + i * 16 + lr) * DB_CS + wc * 64 + ch * 32 + j * 16 + 4 * lg);
+                                       stg + (wr * RH + i * 16 + lro) * DB_CS + wc * 64 + ch * 32 + j * 16 + 4 * lgo);
         __syncthreads();
 #pragma unroll 1
         for (int w = 0; w < 2; w++)
@@ -388,7 +371,7 @@ template <int BM, int BN, int NSTG, bool BF16, int EPV>
 __global__ void __launch_bounds__(256, 2) gemm_dense_tile(DArgs g, EpArgs ep) {
     using T = DTile<BM, BN, NSTG>;
     constexpr int MI = BM / 32, NJ = BN / 32;  // 16 x 16 tiles of a wave's piece
-    __shared__ __align__(16) uint8_t ring[T::LDS(EPV)];
+    __shared__ __align__(1024) uint8_t ring[T::LDS(EPV)];
     const int t = threadIdx.x, lane = t % 64, lr = lane % 16, lg = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(t / 64);
     const int wr = wave / 2, wc = wave % 2;
@@ -398,44 +381,36 @@ __global__ void __launch_bounds__(256, 2) gemm_dense_tile(DArgs g, EpArgs ep) {
     const uint32_t lds0 = lds_addr(ring);
     const uint32_t ksteps = (g.k + 63) / 64, last = ksteps - 1;
 
-    const uint8_t *const abase = (const uint8_t *)(g.a + (size_t)row0 * g.lda);
-    const uint8_t *const bbase = (const uint8_t *)(g.b + (size_t)col0 * g.ldb);
+    const rsrc4_t ra = dense_rsrc(g.a, row0, g.m, g.lda, g.k), rb = dense_rsrc(g.b, col0, g.brows, g.ldb, g.k);
+    const uint32_t lda2 = (uint32_t)g.lda * 2, ldb2 = (uint32_t)g.ldb * 2;
     const uint32_t chunk = (lane % 8) ^ (lane / 8);  // slot lane % 8 of row lane / 8 (mod 8)
-    uint32_t ao[MI], bo[NJ];
-#pragma unroll
-    for (int q = 0; q < MI; q++)
-        ao[q] = (uint32_t)(min((uint32_t)((q * 4 + wave) * 8 + lane / 8), g.m - 1 - row0) * g.lda * 2) + chunk * 16;
-#pragma unroll
-    for (int q = 0; q < NJ; q++)
-        bo[q] = (uint32_t)(min((uint32_t)((q * 4 + wave) * 8 + lane / 8), g.brows - 1 - col0) * g.ldb * 2) + chunk * 16;
+    const uint32_t va = (lane / 8) * lda2 + chunk * 16, vb = (lane / 8) * ldb2 + chunk * 16;
     auto dma = [&](uint32_t step, uint32_t stage) __attribute__((always_inline)) {
         const uint32_t ks = min(step, last), dst = lds0 + stage * T::STAGE + wave * 1024;
-        const uint8_t *ab = abase + (size_t)ks * 128, *bb = bbase + (size_t)ks * 128;
-        if (ks * 64 + 64 <= g.k) {
-#pragma unroll
-            for (int q = 0; q < MI; q++) dma16(ab, ao[q], dst + q * 4096);
-#pragma unroll
-            for (int q = 0; q < NJ; q++) dma16(bb, bo[q], dst + T::A + q * 4096);
-        } else {  // the last step's chunks past K are zeros
+        uint32_t v = va, w = vb;
+        if (ks * 64 + 64 > g.k) {
             const bool in = ks * 64 + chunk * 8 < g.k;
-#pragma unroll
-            for (int q = 0; q < MI; q++) dma16_lane(in ? (const void *)(ab + ao[q]) : (const void *)dense_zeros, dst + q * 4096);
-#pragma unroll
-            for (int q = 0; q < NJ; q++)
-                dma16_lane(in ? (const void *)(bb + bo[q]) : (const void *)dense_zeros, dst + T::A + q * 4096);
+            v = in ? v : OOB;
+            w = in ? w : OOB;
         }
+#pragma unroll
+        for (int q = 0; q < MI; q++) dma16_buf(ra, v, (q * 4 + wave) * 8 * lda2 + ks * 128, dst + q * 4096);
+#pragma unroll
+        for (int q = 0; q < NJ; q++) dma16_buf(rb, w, (q * 4 + wave) * 8 * ldb2 + ks * 128, dst + T::A + q * 4096);
     };
-    const uint32_t f0 = (lg ^ (lr & 7)) << 4;
-    const uint32_t fa = (wr * (BM / 2) + lr) * 128, fb = T::A + (wc * (BN / 2) + lr) * 128;
+    const uint32_t f0 = lr * 128 + ((lg ^ (lr & 7)) << 4);
+    const uint32_t fa = lds0 + wr * (BM / 2) * 128 + f0, fb = lds0 + T::A + wc * (BN / 2) * 128 + f0;
     struct Frags {
         u32x4_t a[MI], b[NJ];
     };
     auto read = [&](uint32_t stage, int kk, Frags &f) __attribute__((always_inline)) {
-        const uint32_t sb = lds0 + stage * T::STAGE + (f0 ^ (kk * 64));
+        const uint32_t sb = stage * T::STAGE;
+        uint32_t ba = sb + (fa ^ (kk * 64)), bb = sb + (fb ^ (kk * 64));
+        asm volatile("" : "+v"(ba), "+v"(bb));  // constant offsets from here
 #pragma unroll
-        for (int i = 0; i < MI; i++) f.a[i] = lds_load<u32x4_t>(sb + fa + i * 2048);
+        for (int i = 0; i < MI; i++) f.a[i] = lds_load<u32x4_t>(ba + i * 2048);
 #pragma unroll
-        for (int j = 0; j < NJ; j++) f.b[j] = lds_load<u32x4_t>(sb + fb + j * 2048);
+        for (int j = 0; j < NJ; j++) f.b[j] = lds_load<u32x4_t>(bb + j * 2048);
     };
     float4_t acc[MI][NJ];
 #pragma unroll
@@ -517,18 +492,18 @@ hipError_t launch_tile(const DArgs &g, const EpArgs &ep, int epv, hipStream_t s)
 // The tile for an m x n x k product: the least of a cost in us, steps of 64
 // depths x (full rounds of the device's compute units x occupancy, each at
 // `full`; a last round of one workgroup a compute unit or fewer at `one`) +
-// `fixed`, with the constants measured on 256 compute units. It gives (us
-// measured, f16, tiles 256x256 / 128x256 / 64x128 / 64x64 / 32x64): 4096^3 107 /
-// 162 / 181 / 218 / 282; 512 x 14336 x 4096 86 / 71 / 84 / 95 / 139; 2048^3 45 /
-// 36 / 26 / 30 / 40; 1000 x 3000 x 2000 45 / 36 / 25 / 29 / 34; 256 x 4096 x
-// 4096 74 / 60 / 37 / 22 / 21; 64 x 512 x 512 15 / - / 6.6 / 5.2 / 4.5.
-// (gemm_kernel, which served these calls before: 197, 95, 47, 60, 80, 12.)
+// `fixed`, with the constants measured on 256 compute units. Measured (us, f16,
+// tiles 256x256 / 128x256 / 64x128 / 64x64 / 32x64): 4096^3 105 / 145 / 181 /
+// 218 / 282; 512 x 14336 x 4096 86 / 64 / 84 / 95 / 139; 2048^3 45 / 34 / 25 / 30
+// / 40; 1000 x 3000 x 2000 45 / 34 / 24 / 29 / 34; 256 x 4096 x 4096 74 / 58 / 36
+// / 20 / 21; 64 x 512 x 512 15 / - / 6.6 / 5.2 / 4.3. (gemm_kernel, which served
+// these calls before: 197, 95, 47, 60, 80, 12.)
 struct DCost {
     uint32_t bm, bn, occ;
     float one, full, fixed;
 };
-constexpr DCost DENSE_TILES[] = {{256, 256, 1, 1.55f, 1.55f, 8.0f},
-                                 {128, 256, 1, 1.10f, 1.10f, 6.0f},
+constexpr DCost DENSE_TILES[] = {{256, 256, 1, 1.50f, 1.50f, 8.0f},
+                                 {128, 256, 1, 0.97f, 0.97f, 6.0f},
                                  {64, 128, 2, 0.53f, 0.70f, 3.0f},
                                  {64, 64, 2, 0.29f, 0.45f, 2.5f},
                                  {32, 64, 3, 0.235f, 0.43f, 2.5f}};

@@ -27,6 +27,19 @@ __device__ __forceinline__ void dma4(const void *sbase, uint32_t voff, uint32_t 
                  "s"(lds)
                  : "memory", "m0");
 }
+// The same through a buffer resource (make_rsrc4): the 16 bytes at voff + soff,
+// zeros where that lies past the resource.
+typedef int rsrc4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ rsrc4_t make_rsrc4(const void *base, uint32_t bytes) {
+    const uint64_t b = (uint64_t)base;
+    return (rsrc4_t){__builtin_amdgcn_readfirstlane((int)b), __builtin_amdgcn_readfirstlane((int)(b >> 32) & 0xFFFF),
+                     __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
+}
+__device__ __forceinline__ void dma16_buf(const rsrc4_t &r, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r),
+                 "s"(soff), "s"(lds)
+                 : "memory", "m0");
+}
 #pragma clang diagnostic pop
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p;
