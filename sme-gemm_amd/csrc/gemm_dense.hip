@@ -40,7 +40,6 @@ namespace smg {
 
 namespace {
 
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 struct DArgs {
@@ -202,7 +201,7 @@ __global__ void __launch_bounds__(DB_NT) gemm_dense_big(DArgs g, EpArgs ep) {
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const uint32_t r = (q * 8 + wave) * 8, row = (r / WR) * (2 * WR) + h * WR + r % WR;
-            dma16_buf(COLS ? rb : ra, v, row * (COLS ? ldb2 : lda2) + ks * 128, dst + q * 8192);
+            dma16_buf(COLS ? rb : ra, v + row * (COLS ? ldb2 : lda2) + ks * 128, dst + q * 8192);
         }
     };
     constexpr std::integral_constant<bool, false> rows;
@@ -394,9 +393,9 @@ __global__ void __launch_bounds__(256, 2) gemm_dense_tile(DArgs g, EpArgs ep) {
             w = in ? w : OOB;
         }
 #pragma unroll
-        for (int q = 0; q < MI; q++) dma16_buf(ra, v, (q * 4 + wave) * 8 * lda2 + ks * 128, dst + q * 4096);
+        for (int q = 0; q < MI; q++) dma16_buf(ra, v + (q * 4 + wave) * 8 * lda2 + ks * 128, dst + q * 4096);
 #pragma unroll
-        for (int q = 0; q < NJ; q++) dma16_buf(rb, w, (q * 4 + wave) * 8 * ldb2 + ks * 128, dst + T::A + q * 4096);
+        for (int q = 0; q < NJ; q++) dma16_buf(rb, w + (q * 4 + wave) * 8 * ldb2 + ks * 128, dst + T::A + q * 4096);
     };
     const uint32_t f0 = lr * 128 + ((lg ^ (lr & 7)) << 4);
     const uint32_t fa = lds0 + wr * (BM / 2) * 128 + f0, fb = lds0 + T::A + wc * (BN / 2) * 128 + f0;
@@ -541,9 +540,10 @@ bool gemm_dense_supported(const DenseGemm &d) {
     const size_t big = (size_t)1 << 31;
     return d.m > 0 && d.n > 0 && d.k >= 64 && d.k % 8 == 0 && d.lda % 8 == 0 && d.ldb % 8 == 0 &&
            d.lda >= (long)d.k && d.ldb >= (long)d.k && ((uintptr_t)d.a & 15) == 0 && ((uintptr_t)d.b & 15) == 0 &&
-           // one 32-bit offset spans a tile's rows; A as gemm_kernel's buffer resource takes it
-           ((d.m - 1) * (size_t)d.lda + d.k) * 2 < big && (size_t)DB * d.lda * 2 < 2 * big &&
-           (size_t)DB * d.ldb * 2 < 2 * big && d.m < big && d.n < big && d.k < big;
+           // a tile's rows and a row's K within 2^31 bytes (past a resource's end
+           // OOB plus that offset still lies past it); A as gemm_kernel takes it
+           ((d.m - 1) * (size_t)d.lda + d.k) * 2 < big && (size_t)(DB + 1) * d.lda * 2 < big &&
+           (size_t)(DB + 1) * d.ldb * 2 < big && d.m < big && d.n < big && d.k < big;
 }
 
 hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hipStream_t s) {

@@ -119,7 +119,6 @@ __device__ __forceinline__ void dma_step(const RArgs &g, const DmaSrc &d, const 
 // column tile, the raw dword and scale (min) of this lane's 8 depths.
 // (32-bit vector types, not arrays of 16-bit values: the fields stay in
 // registers, one element per register)
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 struct Half {
     u32x4_t a[8];
     u32x4_t q, s, mn;

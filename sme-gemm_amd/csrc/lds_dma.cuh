@@ -27,17 +27,18 @@ __device__ __forceinline__ void dma4(const void *sbase, uint32_t voff, uint32_t 
                  "s"(lds)
                  : "memory", "m0");
 }
-// The same through a buffer resource (make_rsrc4): the 16 bytes at voff + soff,
-// zeros where that lies past the resource.
+// The same through a buffer resource (make_rsrc4): the 16 bytes at voff, zeros
+// where that lies past the resource. (The whole offset is the lane's: the
+// range check takes the resource's size less a scalar offset, which would wrap
+// for one past the end.)
 typedef int rsrc4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ rsrc4_t make_rsrc4(const void *base, uint32_t bytes) {
     const uint64_t b = (uint64_t)base;
     return (rsrc4_t){__builtin_amdgcn_readfirstlane((int)b), __builtin_amdgcn_readfirstlane((int)(b >> 32) & 0xFFFF),
                      __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
 }
-__device__ __forceinline__ void dma16_buf(const rsrc4_t &r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r),
-                 "s"(soff), "s"(lds)
+__device__ __forceinline__ void dma16_buf(const rsrc4_t &r, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds)
                  : "memory", "m0");
 }
 #pragma clang diagnostic pop
@@ -62,6 +63,7 @@ __device__ __forceinline__ void barrier_lds() {
     asm volatile("" ::: "memory");
 }
 
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(3))) uint8_t lds_u8_t;
 template <class T>
 __device__ __forceinline__ T lds_load(uint32_t addr) {
