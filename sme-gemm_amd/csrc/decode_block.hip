@@ -25,7 +25,9 @@
 // of squares, split softmax) and exp / tanh are the device's, so results are
 // held to a tolerance against the portable path, not to its bits.
 #include <atomic>
+#include <type_traits>
 
+#include "lds_dma.cuh"
 #include "q4_gemv_core.cuh"
 
 namespace smg {
@@ -893,6 +895,348 @@ __global__ void __launch_bounds__(AP_T) attn_rows_mfma(AttnArgs a) {
         }
 }
 
+// ---------------------------------------------------------------------------
+// The same attention for head dims up to 128, staged by DMA
+// ---------------------------------------------------------------------------
+// attn_rows_dma has attn_rows_mfma's arithmetic. A workgroup of 8 waves takes
+// one KV head and four units of 16 query rows: hg of its query heads (4, 2 or
+// 1, the largest that divides the group) at 4 / hg position tiles. Keys and
+// values go global -> LDS by DMA as they lie (rows of HDM halfs, 16-byte chunks
+// swizzled so that both operands' reads spread over the banks), 128 keys a
+// block, five tiles (of keys or values) in LDS. A wave takes two units and a quarter (32 keys) of every
+// block, so a key or value fragment read from LDS serves 32 query rows:
+//   S^T = K Q^T on v_mfma_f32_16x16x32_f16; O^T += V^T P^T on the same
+//   instruction, whose B operand is S^T's accumulators of two 16-key tiles as
+//   they stand (lane l: row l % 16, keys 4 (l / 16) .. + 3 of each), and whose A
+//   operand comes from the row-major values by the transposing LDS read
+//   (ds_read_b64_tr_b16: 4 keys x 16 depths a 16-lane group) with the same key
+//   order.
+// A row's running max only moves when a score passes it by more than 8 in
+// log2 (the probabilities stay below 2^8, as exact in f16 as below 1), so the
+// usual block has no cross-lane step and no rescale; the row sums stay per
+// lane until the end, where the four key quarters of a unit are merged through
+// LDS. Masks (scores, and values past the unit's last position, so that no
+// row's probability of zero meets them) only where a wave's keys reach the
+// unit's own positions.
+// What bounds it: about 130 vector instructions (16 of them 2^x) and 32 products
+// a wave and block, two waves a SIMD, one barrier a block. Measured (us, one
+// MI355X, q's rounding pass included; attn_rows_mfma, one wave a SIMD with 160
+// KB of LDS traffic a 64-key block, before): 512 rows after 4096 positions, 32
+// heads of 128 over 8 KV heads 136 -> 69, over 32 KV heads 373 -> 68; 1024 rows
+// after 8192 370 -> 226; 32 rows after 8192, 12 heads of 64, 145 -> 55. Kept out:
+// wave groups one phase apart with a barrier between scores and values (87),
+// both in lockstep phases (77): the barrier's wait exceeds what it overlaps.
+constexpr int AD_T = 512, AD_KB = 128, AD_U = 4;  // threads, keys a block, units
+constexpr float AD_LOW = -1e30f;                  // below every finite score
+
+template <int HDM>
+struct AttnDma {
+    static constexpr int CH = HDM / 8;              // 16-byte chunks a row
+    static constexpr int ROWB = HDM * 2;            // bytes a row
+    static constexpr int TILE = AD_KB * ROWB;       // keys (values) of a block
+    static constexpr int NT = 5;                    // tiles in LDS
+    static constexpr int NI = TILE / (8 * 1024);    // DMA instructions a wave, keys (values)
+    static constexpr int KK = HDM / 32, DT = HDM / 16;
+    // chunk c of row r sits at slot c ^ ksw(r) (keys), c ^ vsw(r) (values): the
+    // 16 rows of a key fragment, and the 8 rows x 2 chunks of half a wave's
+    // transposing read, take distinct 16-byte bank columns
+    static __device__ __forceinline__ uint32_t ksw(uint32_t r) { return HDM == 128 ? r & 15 : (r >> 1) & 7; }
+    static __device__ __forceinline__ uint32_t vsw(uint32_t r) { return HDM == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
+};
+
+template <int HDM>
+__global__ void __launch_bounds__(AD_T) attn_rows_dma(AttnArgs a, uint32_t hg) {
+    using T = AttnDma<HDM>;
+    constexpr int KK = T::KK, DT = T::DT;
+    __shared__ __align__(1024) uint8_t smem[T::NT * T::TILE];
+    const int t = threadIdx.x, lane = t % 64, r16 = lane % 16, g4 = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(t / 64), up = wave & 1, kq = wave >> 1;
+    // consecutive workgroups take one position block's head chunks, so the
+    // workgroups of one KV head share an XCD's L2 when their count is a
+    // multiple of 8
+    const uint32_t hch = a.group / hg, ny = (a.heads / a.group) * hch, yc = blockIdx.x % ny;
+    const uint32_t kvh = yc / hch, hc0 = (yc % hch) * hg, tiles = AD_U / hg, tile0 = (blockIdx.x / ny) * tiles;
+    const uint32_t nkeys = a.len + min((tile0 + tiles) * 16, a.rows) - 1;  // the last position's prefix
+    const uint32_t nblk = (nkeys + AD_KB - 1) / AD_KB;
+
+    // the wave's units: head, this lane's row, the first row's keys (fewer need
+    // no mask) and the last row's (0: no rows)
+    uint32_t head[2], row[2], first[2], ukeys[2];
+    u32x4_t qf[2][KK];
+    const rsrc_t qr = make_rsrc(a.q, a.rows * a.heads * a.hd * 2u);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t u = 2 * up + j, p0 = (tile0 + u / hg) * 16;
+        head[j] = kvh * a.group + hc0 + u % hg;
+        row[j] = p0 + r16;
+        first[j] = a.len + p0;
+        ukeys[j] = p0 < a.rows ? a.len + min(p0 + 16, a.rows) - 1 : 0;
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) {
+            const uint32_t d = 32u * kk + 8u * g4;
+            qf[j][kk] = __builtin_bit_cast(
+                u32x4_t, bload16(qr, row[j] < a.rows && d < a.hd ? ((row[j] * a.heads + head[j]) * a.hd + d) * 2u : OOB));
+        }
+    }
+
+    // DMA: instruction i moves rows (8 i + wave) RPI .. of the block (RPI rows of
+    // CH chunks); rows past nkeys and chunks past hd read zeros
+    constexpr int RPI = 64 / T::CH;
+    const uint32_t ld2 = a.ld * 2, rl = wave * RPI + lane / T::CH, slot = lane % T::CH;
+    const uint32_t kc = slot ^ T::ksw(rl), vc = slot ^ T::vsw(rl);  // (8 RPI rows apart: the same swizzle)
+    const uint32_t base = kvh * a.hd * 2 + rl * ld2;
+    const uint32_t ko = kc * 8 < a.hd ? base + kc * 16 : OOB, vo = vc * 8 < a.hd ? base + vc * 16 : OOB;
+    const rsrc4_t kr = make_rsrc4(a.k, nkeys * ld2), vr = make_rsrc4(a.v, nkeys * ld2);
+    const uint32_t lds0 = lds_addr(smem);
+    // Tile seq of the sequence keys 0, values 0, keys 1, values 1, ... goes to
+    // slot seq % NT (a tile past the last block's reloads one into a free slot).
+    auto slot_of = [&](uint32_t seq) __attribute__((always_inline)) { return lds0 + seq % T::NT * T::TILE; };
+    auto dma = [&](uint32_t seq) __attribute__((always_inline)) {
+        const uint32_t dst = slot_of(seq) + wave * 1024, b = min(seq / 2, nblk - 1);
+        const uint32_t o0 = b * AD_KB * ld2, step = 8 * RPI * ld2;
+        if (seq & 1) {  // uniform
+#pragma unroll
+            for (int i = 0; i < T::NI; i++) dma16_buf(vr, vo + (o0 + i * step), dst + i * 8192);
+        } else {
+#pragma unroll
+            for (int i = 0; i < T::NI; i++) dma16_buf(kr, ko + (o0 + i * step), dst + i * 8192);
+        }
+    };
+
+    // this lane's fragment addresses in a tile: key row r16 of the wave's first
+    // tile, chunk g4; the transposing read's row 4 g4 + (lane % 16) / 4, depth 4
+    // (lane % 4) (the chunk's bit 0 is lane bit 1)
+    const uint32_t kf = (kq * 32 + r16) * T::ROWB, ks = T::ksw(r16);  // row % 16 is r16
+    const uint32_t vrow = kq * 32 + 4 * g4 + r16 / 4;
+    const uint32_t vf = vrow * T::ROWB + (lane & 1) * 8, vs = T::vsw(vrow);  // rows + 16: the same
+
+    float4_t o[2][DT];
+    float m2[2] = {AD_LOW, AD_LOW}, l[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[j][dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    constexpr float LOG2E = 1.4426950408889634f;
+
+    // S^T of the wave's 32 keys (of the block in the tile at LDS address sb) for
+    // both units.
+    auto scores = [&](uint32_t sb, float4_t (&sc)[2][2]) __attribute__((always_inline)) {
+        u32x4_t ka[KK][2];
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+                ka[kk][kt] = lds_load<u32x4_t>(sb + kf + kt * 16 * T::ROWB + (((kk * 4 + g4) ^ ks) << 4));
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) sc[0][kt] = sc[1][kt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    sc[j][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ka[kk][kt]),
+                                                                       __builtin_bit_cast(half8_t, qf[j][kk]), sc[j][kt],
+                                                                       0, 0, 0);
+    };
+    // The running max and sum, and the probabilities of the scores of the 32
+    // keys from k0 on. DIAG: keys past a row's own position are masked.
+    auto softmax = [&](float4_t (&sc)[2][2], uint32_t k0, half8_t (&pf)[2], auto diag_c) __attribute__((always_inline)) {
+        constexpr bool DIAG = decltype(diag_c)::value;
+        float mx[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (DIAG) {
+                const uint32_t lim = a.len + row[j];
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (k0 + 16 * (e / 4) + 4 * g4 + e % 4 >= lim) sc[j][e / 4][e % 4] = -INFINITY;
+            }
+            mx[j] = sc[j][0][0];
+#pragma unroll
+            for (int e = 1; e < 8; e++) mx[j] = fmaxf(mx[j], sc[j][e / 4][e % 4]);
+        }
+        const float over = fmaxf(__builtin_fmaf(mx[0], LOG2E, -m2[0]), __builtin_fmaf(mx[1], LOG2E, -m2[1]));
+        if (__builtin_amdgcn_ballot_w64(over > 8.0f) != 0) {
+            // some row's max moved: the rows' new max over their four lanes
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                mx[j] = fmaxf(mx[j], xor_lanes(mx[j], 16));
+                mx[j] = fmaxf(mx[j], xor_lanes(mx[j], 32));
+                const float mn = fmaxf(m2[j], mx[j] * LOG2E);
+                const float alpha = m2[j] == mn ? 1.0f : __builtin_amdgcn_exp2f(m2[j] - mn);
+                m2[j] = mn;
+                l[j] = l[j] * alpha;
+                // (in place: otherwise the merge of the two paths copies every o)
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        float x = o[j][dt][v];
+                        asm volatile("v_mul_f32 %0, %1, %0" : "+v"(x) : "v"(alpha));
+                        o[j][dt][v] = x;
+                    }
+            }
+        }
+        // e^(x - m) as the hardware 2^(x log2 e - m2)
+        typedef float f32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            half2_t h[4];
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const f32x2_t p = {__builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][e / 4][e % 4], LOG2E, -m2[j])),
+                                   __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][e / 4][e % 4 + 1], LOG2E, -m2[j]))};
+                l[j] = l[j] + (p[0] + p[1]);
+                h[e / 2] = __builtin_convertvector(p, half2_t);
+            }
+            const half4_t h0 = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3);
+            const half4_t h1 = __builtin_shufflevector(h[2], h[3], 0, 1, 2, 3);
+            pf[j] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    // O^T += V^T P^T: 16 depths x 32 keys a product. DIAG: values past a unit's
+    // last position are zeros.
+    typedef short s4_t __attribute__((ext_vector_type(4)));
+    typedef short s8_t __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s4_t lds_s4_t;
+    auto values = [&](uint32_t sb, uint32_t k0, const half8_t (&pf)[2], auto diag_c) __attribute__((always_inline)) {
+        constexpr bool DIAG = decltype(diag_c)::value;
+        s4_t vv[DT][2];
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+            const uint32_t va = sb + vf + (((2 * dt + (r16 % 4) / 2) ^ vs) << 4);
+            vv[dt][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t *)(lds_u8_t *)(uintptr_t)va);
+            vv[dt][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t *)(lds_u8_t *)(uintptr_t)(va + 16 * T::ROWB));
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                s4_t x[2] = {vv[dt][0], vv[dt][1]};
+                if constexpr (DIAG) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (k0 + 16 * (e / 4) + 4 * g4 + e % 4 >= ukeys[j]) x[e / 4][e % 4] = 0;
+                }
+                const s8_t v8 = __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                o[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, v8), pf[j], o[j][dt], 0, 0,
+                                                                  0);
+            }
+    };
+    // Step b scores block b and multiplies block b - 1's values, whose products
+    // fill the matrix cores beside the other wave's softmax; its start ends the
+    // use of tiles up to 2b - 2, whose slots take tiles 2b + 2 and 2b + 3.
+#pragma unroll
+    for (int i = 0; i < 4; i++) dma(i);
+    // the queries are waited for here, once (inside the loop the compiler's wait
+    // for them would drain the DMA)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) asm volatile("" : "+v"(qf[j][kk]));
+    half8_t pf[2];
+    float4_t sc[2][2];
+    constexpr std::integral_constant<bool, false> inner;
+    constexpr std::integral_constant<bool, true> edge;
+    const uint32_t kw = kq * 32;  // the wave's keys of a block
+    // tiles 2b and 2b - 1 have landed for every wave (2b + 1 is younger), and
+    // every wave has read step b - 1's
+    auto start = [&](uint32_t b) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        wait_vm<T::NI>();
+        barrier_lds();
+        dma(2 * b + 2);
+        dma(2 * b + 3);
+    };
+    {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        wait_vm<3 * T::NI>();
+        barrier_lds();
+        scores(slot_of(0), sc);
+        softmax(sc, kw, pf, edge);
+    }
+    // blocks whose keys every row of the workgroup attends to, then the rest (a
+    // wave's keys past all its rows' are masked, and their values zeros)
+    const uint32_t nfull = min(nblk, (a.len + tile0 * 16) / AD_KB);
+    uint32_t b = 1;
+    for (; b < nfull; b++) {
+        start(b);
+        scores(slot_of(2 * b), sc);
+        values(slot_of(2 * b - 1), (b - 1) * AD_KB + kw, pf, inner);
+        softmax(sc, b * AD_KB + kw, pf, inner);
+    }
+    for (; b < nblk; b++) {
+        start(b);
+        scores(slot_of(2 * b), sc);
+        values(slot_of(2 * b - 1), (b - 1) * AD_KB + kw, pf, edge);
+        softmax(sc, b * AD_KB + kw, pf, edge);
+    }
+    wait_vm<0>();
+    barrier_lds();
+    values(slot_of(2 * nblk - 1), (nblk - 1) * AD_KB + kw, pf, edge);
+    // Merge the key quarters: 2 into 0 and 3 into 1, then 1 into 0. A wave's
+    // state is its lanes' o (16 bytes a lane and depth tile) and its rows' (m2,
+    // l), the same lanes in every quarter.
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        l[j] = l[j] + xor_lanes(l[j], 16);
+        l[j] = l[j] + xor_lanes(l[j], 32);
+    }
+    constexpr int XW = 2 * DT * 1024 + 2 * 512;  // bytes a wave hands over
+    static_assert(4 * XW <= T::NT * T::TILE, "the exchange exceeds the tiles");
+#pragma unroll
+    for (int round = 0; round < 2; round++) {
+        const int give = round == 0 ? 2 : 1;  // quarters [give, 2 give) hand over
+        __syncthreads();
+        uint8_t *x = smem + ((kq % give) * 2 + up) * XW;
+        if (kq >= give && kq < 2 * give) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) *(float4_t *)(x + ((j * DT + dt) * 64 + lane) * 16) = o[j][dt];
+                *(float2 *)(x + 2 * DT * 1024 + (j * 64 + lane) * 8) = make_float2(m2[j], l[j]);
+            }
+        }
+        __syncthreads();
+        if (kq < give) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float2 ml = *(const float2 *)(x + 2 * DT * 1024 + (j * 64 + lane) * 8);
+                const float mn = fmaxf(m2[j], ml.x);
+                const float wa = m2[j] == mn ? 1.0f : __builtin_amdgcn_exp2f(m2[j] - mn);
+                const float wb = ml.x == mn ? 1.0f : __builtin_amdgcn_exp2f(ml.x - mn);
+                m2[j] = mn;
+                l[j] = l[j] * wa + ml.y * wb;
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) {
+                    const float4_t ob = *(const float4_t *)(x + ((j * DT + dt) * 64 + lane) * 16);
+                    o[j][dt] = o[j][dt] * wa + ob * wb;
+                }
+            }
+        }
+    }
+    if (kq != 0) return;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (row[j] >= a.rows) continue;
+        const size_t ob = ((size_t)row[j] * a.heads + head[j]) * a.hd;
+        const float inv = 1.0f / l[j];
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+            const uint32_t d = 16u * dt + 4u * g4;
+            if (d >= a.hd) continue;  // hd is a multiple of 8
+            const float4_t val = o[j][dt] * inv;
+            if (a.f16_out)
+                *(uint2 *)((uint16_t *)a.out + ob + d) =
+                    make_uint2((uint32_t)f32_to_f16(val[0]) | ((uint32_t)f32_to_f16(val[1]) << 16),
+                               (uint32_t)f32_to_f16(val[2]) | ((uint32_t)f32_to_f16(val[3]) << 16));
+            else
+                *(float4_t *)((float *)a.out + ob + d) = val;
+        }
+    }
+}
+
 // m rows of the qkv projection (an f16 GEMM output in the fused QKV store's
 // device column order: a 16-column tile holds depths 8q..8q+7 and
 // half+8q..half+8q+7 of one head, each RoPE pair in lanes c, c ^ 8) to the
@@ -1057,6 +1401,14 @@ hipError_t launch_attention(const AttnArgs &a0, void *out, bool f16_out, hipStre
         if ((size_t)a.rows * a.heads * a.hd * 2 >= ((size_t)1 << 31)) return hipErrorInvalidValue;
         a.out = out;
         a.f16_out = f16_out ? 1u : 0u;
+        if (a.hd <= 128 && (last + AD_KB) * a.ld * 2 < ((size_t)1 << 31) && a.ld % 8 == 0 &&
+            (((uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.q | (uintptr_t)a.out) & 15) == 0) {
+            const uint32_t hg = a.group % 4 == 0 ? 4 : a.group % 2 == 0 ? 2 : 1, tr = 16 * AD_U / hg;
+            const dim3 dgrid(((a.rows + tr - 1) / tr) * (a.heads / hg));
+            if (a.hd <= 64) hipLaunchKernelGGL(attn_rows_dma<64>, dgrid, dim3(AD_T), 0, s, a, hg);
+            else hipLaunchKernelGGL(attn_rows_dma<128>, dgrid, dim3(AD_T), 0, s, a, hg);
+            return hipGetLastError();
+        }
         const dim3 grid(((a.rows + AP_BR - 1) / AP_BR) * (a.heads / a.group) * a.hchunks);
         if (a.hd <= 64) hipLaunchKernelGGL(attn_rows_mfma<64>, grid, dim3(AP_T), 0, s, a);
         else if (a.hd <= 128) hipLaunchKernelGGL(attn_rows_mfma<128>, grid, dim3(AP_T), 0, s, a);

@@ -853,3 +853,48 @@ def test_layer_norm_block_gpt2_style(smg, orc, rows, bias):
     ck, cv = inp["cache_k"].copy(), inp["cache_v"].copy()
     _rows_vs_oracle(orc, p, x0, x.cpu().numpy().reshape(rows, d), ck, cv, keys, vals, past, rows, d, H * hd, ffn,
                     set(range(rows)))
+
+
+# The DMA-staged causal attention (head dims up to 128, rows >= 32): the query
+# heads a workgroup takes (4, 2, 1) at position tiles that end inside its last
+# tile, key blocks of 128 whose last one is short, padded head dims, prefixes
+# that end on and beside a block.
+@pytest.mark.parametrize("heads,kv_heads,hd,start,rows", [
+    (8, 2, 128, 96, 32), (8, 2, 128, 97, 33), (4, 2, 64, 0, 70), (6, 2, 80, 300, 47), (3, 3, 64, 1, 65),
+    (5, 5, 128, 127, 129), (12, 1, 8, 128, 40), (2, 1, 16, 255, 64), (4, 4, 120, 500, 31 + 64)])
+def test_causal_rows_dma_tiles(smg, heads, kv_heads, hd, start, rows):
+    """Against float64 softmax attention on the f16-rounded q * scale, whose
+    probabilities the kernel rounds to f16 (2^-11 relative each): within 2e-3
+    (1 + max|v|). Scores grow along the keys, so the running max moves often."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(heads * 1000 + rows)
+    ln, ql, ld = start + rows, heads * hd, kv_heads * hd
+    q = torch.randn(rows, ql, generator=g, device="cuda")
+    k = torch.randn(ln, ld, generator=g, device="cuda")
+    k = (k * torch.linspace(0.1, 4.0, ln, device="cuda")[:, None]).half()
+    v = torch.randn(ln, ld, generator=g, device="cuda").half()
+    out = torch.full_like(q, float("nan"))
+    scale = hd ** -0.5
+    smg.attention_kv_causal_f16(q, k, v, start, rows, heads, kv_heads, hd, scale, out)
+    qs = (q * scale).half().double()
+    mask = torch.arange(ln, device="cuda")[None] > start + torch.arange(rows, device="cuda")[:, None]
+    for h in range(heads):
+        j = h // (heads // kv_heads)
+        s = qs[:, h * hd:(h + 1) * hd] @ k[:, j * hd:(j + 1) * hd].double().t().contiguous()
+        w = torch.softmax(s.masked_fill(mask, -float("inf")), 1) @ v[:, j * hd:(j + 1) * hd].double().contiguous()
+        err = (out[:, h * hd:(h + 1) * hd].double() - w).abs().max().item()
+        assert err <= 2e-3 * (1 + v.abs().max().item()), (h, err)
+
+
+def test_causal_rows_dma_keeps_later_positions_out(smg):
+    """NaN keys and values at a later position reach only the rows that attend
+    to it or share its 16-row tile (no other tile multiplies them)."""
+    import torch
+    heads, hd, start, rows = 2, 64, 40, 96
+    q = torch.randn(rows, heads * hd, device="cuda")
+    k, v = (torch.randn(start + rows, heads * hd, device="cuda").half() for _ in range(2))
+    k[start + 50], v[start + 50] = float("nan"), float("nan")
+    out = torch.empty_like(q)
+    smg.attention_kv_causal_f16(q, k, v, start, rows, heads, heads, hd, hd ** -0.5, out)
+    assert bool(torch.isfinite(out[:48]).all())
+    assert bool(out[50:].isnan().all())
