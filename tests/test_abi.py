@@ -366,3 +366,18 @@ def test_host_slice_arrays_in_the_mirror():
     assert smg._same_side(FakeDev(), FakeDev()) is True
     with pytest.raises(ValueError, match="host arrays or all device tensors"):
         smg._same_side(y, FakeDev())
+
+
+def test_packed_descriptor_is_desc():
+    """The packed form a call passes holds desc()'s bytes (the node pointer
+    aside), for every operand class, a stride and a trailing activation."""
+    import smegemm as smg
+    t, r, c = (np.arange(x, dtype=np.uint16) for x in (60, 6, 10))
+    ep = smg.Epilogue().mul_scalar(0.5).add_row(r).mul_col(c).add_tensor(t).max_tensor(t, ld=10).elu(0.3).silu()
+    d, keep = ep.desc(10)
+    addr, keep2 = ep.packed(10)
+    got = C.cast(addr, C.POINTER(smg.EpDesc16)).contents
+    assert got.n_nodes == d.n_nodes == 7
+    size = C.sizeof(smg.EpNode) * 7
+    assert C.string_at(got.nodes, size) == C.string_at(d.nodes, size)
+    assert smg.Epilogue().packed(10) == (None, [])
