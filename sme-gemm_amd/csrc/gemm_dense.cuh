@@ -524,7 +524,7 @@ int dense_pick(size_t m, size_t n, size_t k) {
     return best;
 }
 template <bool BF16>
-hipError_t launch_shape(const DArgs &g, const EpArgs &ep, int epv, hipStream_t s) {
+hipError_t launch_dense_shape(const DArgs &g, const EpArgs &ep, int epv, hipStream_t s) {
     switch (dense_pick(g.m, g.n, g.k)) {
     case 0: return launch_big<256, BF16>(g, ep, epv, s);
     case 1: return launch_big<128, BF16>(g, ep, epv, s);
@@ -567,7 +567,7 @@ hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hi
     g.act = pk.act;
     g.act_alpha = pk.alpha;
     const int epv = g.st.add_dst ? 0 : pk.v;
-    return bf16 ? launch_shape<true>(g, ep, epv, s) : launch_shape<false>(g, ep, epv, s);
+    return bf16 ? launch_dense_shape<true>(g, ep, epv, s) : launch_dense_shape<false>(g, ep, epv, s);
 }
 
 }  // namespace smg

@@ -658,3 +658,9 @@ hipError_t launch_q4_dequant_dense(const WDev &q4, uint16_t *dense, bool to_bf16
 }
 
 }  // namespace smg
+
+// The DMA-staged GEMMs, part of this translation unit: launch_gemm's dense
+// kernels, and the low-bit int8 one, whose arguments are not preloaded as
+// lowbit_gemv.hip's are.
+#include "gemm_dense.cuh"
+#include "lowbit_gemm.cuh"

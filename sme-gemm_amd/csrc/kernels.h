@@ -71,7 +71,7 @@ size_t lowbit_scratch_bytes(const WDev &w, size_t m, const EpArgs *ep = nullptr,
 hipError_t launch_lowbit_gemv(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs,
                               const EpArgs &ep, void *scratch, size_t scratch_bytes, hipStream_t s);
 
-// The many-row form (lowbit_gemm.hip): from LOWBIT_GEMM_ROWS rows, blocks of
+// The many-row form (lowbit_gemm.cuh): from LOWBIT_GEMM_ROWS rows, blocks of
 // 64, 128 or 256. lowbit_gemm_bytes is its scratch, 0 where it does not serve.
 constexpr size_t LOWBIT_GEMM_ROWS = 9;
 size_t lowbit_gemm_bytes(const WDev &w, size_t m);
@@ -94,7 +94,7 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
 hipError_t launch_pack_dense_strided(const uint16_t *rhs, long rhs_rs, long rhs_cs, size_t n, size_t k,
                                      size_t n_pad, size_t k_pad, uint16_t *dense, hipStream_t s);
 
-// The dense GEMM over K-contiguous operands (gemm_dense.hip): A [m][lda], B
+// The dense GEMM over K-contiguous operands (gemm_dense.cuh): A [m][lda], B
 // [n][ldb] (brows >= n rows can be read), C[i,j] at dst[i*dst_rs + j*dst_cs].
 // read_dst: with no graph alpha * C + beta * A@B with one rounding, with one
 // alpha * C added after it.
