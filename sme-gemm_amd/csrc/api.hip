@@ -463,6 +463,16 @@ int make_dense(int kind, const uint16_t *rhs, size_t n, size_t k, long rs, long 
     return SMG_OK;
 }
 
+// Whether the stream is being captured into a graph (then no call allocates).
+bool stream_capturing(void *stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // ---- one host-pointer call ---------------------------------------------------
 // Stages lhs and epilogue operands, runs `launch` on the thread's stream, and
 // copies dst back only after everything succeeded.
@@ -1446,9 +1456,17 @@ static int packed_host(bool bf16, size_t m, size_t n, size_t k, uint16_t *dst, l
     // call's scratch, and the graph's pass adds alpha * old C (the store's
     // add_dst step)
     const bool tail_add = read_dst && ep && ep->n_nodes > (uint32_t)EP_FUSED;
+    // (the staged copy of A is 256-byte aligned)
+    const size_t ab = tail_add ? 0 : dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs);
     return host_call(bf16 ? "gemm_gpu_b16b16_run_packed" : "gemm_gpu_f16f16_run_packed", b->device,
-                     m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, lhs_elems, ep, tail_add ? m * n * 2 : 0,
+                     m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, lhs_elems, ep, tail_add ? m * n * 2 : ab,
                      [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
+                         if (ab) {
+                             const hipError_t e = launch_gemm_pack_a(d, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta,
+                                                                     p.fused, bf16, (uint16_t *)sc, s, read_dst != 0,
+                                                                     alpha);
+                             return e == hipSuccess ? plan_tail(p, dd, dst_cs, dst_rs, m, n, bf16, s) : e;
+                         }
                          if (tail_add) {
                              uint16_t *prod = (uint16_t *)sc;
                              const hipError_t e = launch_gemm(d, m, prod, 1, (long)n, dl, lhs_cs, lhs_rs, beta,
@@ -1535,11 +1553,13 @@ static int run_host(bool bf16, const char *name, size_t m, size_t n, size_t k, u
     const size_t dst_elems = footprint(m, dst_rs, n, dst_cs);
     const bool dense_out = (dst_cs == 1 && (size_t)dst_rs == n) || (dst_rs == 1 && (size_t)dst_cs == m);
     const float alpha = half_bits_to_float(alpha_bits, bf16), beta = half_bits_to_float(beta_bits, bf16);
+    // scratch: the packed B, then the packed A where it is needed, then B as given
+    const size_t ab = dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs), raw_at = dense_bytes + round_up(ab, 256);
     return host_call(name, device, m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, footprint(m, lhs_rs, k, lhs_cs),
-                     nullptr, dense_bytes + rhs_elems * 2,
+                     nullptr, raw_at + rhs_elems * 2,
                      [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
                          const EpArgs &ea = p.fused;  // no op-graph on these entry points
-                         uint16_t *dense = (uint16_t *)sc, *raw = (uint16_t *)((uint8_t *)sc + dense_bytes);
+                         uint16_t *dense = (uint16_t *)sc, *raw = (uint16_t *)((uint8_t *)sc + raw_at);
                          if (rhs_elems) {
                              const hipError_t e = hipMemcpyAsync(raw, rhs, rhs_elems * 2, hipMemcpyHostToDevice, s);
                              if (e != hipSuccess) return e;
@@ -1553,6 +1573,10 @@ static int run_host(bool bf16, const char *name, size_t m, size_t n, size_t k, u
                          if (e != hipSuccess) return e;
                          WDev w = d;
                          w.dense = dense;
+                         if (ab)
+                             return launch_gemm_pack_a(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16,
+                                                       (uint16_t *)((uint8_t *)sc + dense_bytes), s, read_dst != 0,
+                                                       alpha);
                          return launch_gemm(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16, s,
                                             read_dst != 0, alpha);
                      });
@@ -1609,7 +1633,16 @@ int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long
     d.k = k;
     d.n_pad = round_up(n, 128);
     d.k_pad = round_up(k ? k : 1, 64);
-    uint16_t *dense = (uint16_t *)dev_pool().get(device, stream, d.n_pad * d.k_pad * 2);
+    // B packed, and A where gemm_dense cannot read it (left where it is if only
+    // B's share can be had)
+    const size_t bb = round_up(d.n_pad * d.k_pad * 2, 256);
+    size_t ab = dense_pack_a_bytes(d, m, lhs, lhs_cs, lhs_rs);
+    if (ab && stream_capturing(stream) && !dev_pool().find(device, stream, bb + ab)) ab = 0;
+    uint16_t *dense = (uint16_t *)dev_pool().get(device, stream, bb + ab);
+    if (!dense && ab) {
+        ab = 0;
+        dense = (uint16_t *)dev_pool().get(device, stream, bb);
+    }
     if (!dense) return fail(SMG_ENOMEM, "smg_gemm_run_dev: scratch hipMalloc");
     hipError_t e = launch_pack_dense_strided(rhs, rhs_rs, rhs_cs, n, k, d.n_pad, d.k_pad, dense,
                                              (hipStream_t)stream);
@@ -1617,8 +1650,10 @@ int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long
         d.dense = dense;
         EpArgs ea = {};
         const bool b = bf16 != 0;
-        e = launch_gemm(d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ea, b, (hipStream_t)stream,
-                        read_dst != 0, alpha);
+        e = ab ? launch_gemm_pack_a(d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ea, b, dense + bb / 2,
+                                    (hipStream_t)stream, read_dst != 0, alpha)
+               : launch_gemm(d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ea, b, (hipStream_t)stream,
+                             read_dst != 0, alpha);
     }
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_gemm_run_dev", e);
 }
@@ -1759,9 +1794,17 @@ int smg_packed_matmul_dev(size_t m, const smg_weights *b, uint16_t *dst, long ds
     EpPlan ep_p;
     if ((rc = ep_plan(ep, &ep_p, b->d.n))) return rc;
     if ((rc = check_dev_ptrs("smg_packed_matmul_dev", b->device, stream, ep_p, {dst, lhs}))) return rc;
-    hipError_t e = launch_gemm(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs,
-                               half_bits_to_float(beta_bits, bf16 != 0), ep_p.fused, bf16 != 0,
-                               (hipStream_t)stream);
+    // A packed into the stream's scratch where gemm_dense cannot read it; without
+    // the scratch (none to be had, or none yet while the stream is captured)
+    // the product reads A as it is
+    const float beta = half_bits_to_float(beta_bits, bf16 != 0);
+    const size_t ab = dense_pack_a_bytes(b->d, m, lhs, lhs_cs, lhs_rs);
+    void *ap = nullptr;
+    if (ab) ap = stream_capturing(stream) ? dev_pool().find(b->device, stream, ab) : dev_pool().get(b->device, stream, ab);
+    hipError_t e = ap ? launch_gemm_pack_a(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
+                                           (uint16_t *)ap, (hipStream_t)stream)
+                      : launch_gemm(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
+                                    (hipStream_t)stream);
     if (e == hipSuccess) e = plan_tail(ep_p, dst, dst_cs, dst_rs, m, b->d.n, bf16 != 0, (hipStream_t)stream);
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_packed_matmul_dev", e);
 }

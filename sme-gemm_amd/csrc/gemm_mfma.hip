@@ -566,6 +566,32 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
     }
 }
 
+// A dense product whose A gemm_dense cannot read where it is (K not a multiple
+// of 8, rows not 16-byte aligned, a column stride): A is packed as B is, K zero
+// padded to B's k_pad, and the product runs over k_pad. gemm_kernel reads such
+// an A element by element. Measured with a prepacked B (us, the packing of A
+// included): 3000 x 500 x 3001 173 -> 41, 61 x 499 x 523 28 -> 7.8, one row x 4096
+// x 4097 122 -> 18.
+size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs) {
+    if ((w.kind != W_F16 && w.kind != W_BF16) || m == 0 || w.n == 0 || w.k == 0 || lhs_cs < 0 || lhs_rs < 0) return 0;
+    const size_t big = (size_t)1 << 31;
+    const size_t fp = ((m - 1) * (size_t)lhs_rs + (w.k - 1) * (size_t)lhs_cs + 1) * 2, rows = (m + 31) / 32 * 32;
+    if (fp >= big || rows * w.k_pad * 2 >= big || rows / 32 > 65535) return 0;
+    const DenseGemm d = {lhs, w.dense, nullptr, m, w.n, w.k, w.n_pad, lhs_rs, (long)w.k_pad, 1, 1, 1.0f, 0.0f, false};
+    if (lhs_cs == 1 && gemm_dense_supported(d)) return 0;
+    return rows * w.k_pad * 2;
+}
+hipError_t launch_gemm_pack_a(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
+                              long lhs_cs, long lhs_rs, float beta, const EpArgs &ep, bool bf16, uint16_t *scratch,
+                              hipStream_t s, bool read_dst, float alpha) {
+    const hipError_t e =
+        launch_pack_dense_strided(lhs, lhs_cs, lhs_rs, m, w.k, (m + 31) / 32 * 32, w.k_pad, scratch, s);
+    if (e != hipSuccess) return e;
+    WDev p = w;
+    p.k = w.k_pad;
+    return launch_gemm(p, m, dst, dst_cs, dst_rs, scratch, 1, (long)w.k_pad, beta, ep, bf16, s, read_dst, alpha);
+}
+
 // A strided k x n B into the dense layout, 32 x 32 blocks through LDS: the
 // reads run along whichever of B's two strides is 1 when the block's threads
 // walk j (a row-major B) and the writes along the dense column's K.
@@ -588,11 +614,37 @@ __global__ void __launch_bounds__(256) pack_dense_strided(const uint16_t *rhs, l
         if (l < k_pad) dense[(size_t)j * k_pad + l] = tile[tx][ty + 8 * r];
     }
 }
+// The same for a B whose columns' K is contiguous (rhs_rs = 1): whole columns
+// copied and zero padded, 8 depths a thread, consecutive threads along K: read
+// 32 x 32 at a time as above, each load of a wave would touch 32 columns.
+__global__ void __launch_bounds__(256) pack_dense_columns(const uint16_t *rhs, long rhs_cs, uint32_t n, uint32_t k,
+                                                          uint32_t n_pad, uint32_t k_pad, uint16_t *dense) {
+    const uint32_t kc = k_pad / 8;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)n_pad * kc) return;
+    const uint32_t j = (uint32_t)(i / kc), l = (uint32_t)(i % kc) * 8;
+    uint32_t w[4] = {0, 0, 0, 0};
+    if (j < n) {
+        const uint16_t *src = rhs + (size_t)j * rhs_cs + l;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            if (l + e < k) w[e / 2] |= (uint32_t)src[e] << (16 * (e % 2));
+    }
+    *(uint4 *)(dense + (size_t)j * k_pad + l) = make_uint4(w[0], w[1], w[2], w[3]);
+}
 }  // namespace
 
 hipError_t launch_pack_dense_strided(const uint16_t *rhs, long rhs_rs, long rhs_cs, size_t n, size_t k,
                                      size_t n_pad, size_t k_pad, uint16_t *dense, hipStream_t s) {
     if (n_pad % 32 || k_pad % 32 || n > n_pad || k > k_pad) return hipErrorInvalidValue;
+    if (rhs_rs == 1 && k_pad % 8 == 0) {
+        const size_t blocks = (n_pad * (k_pad / 8) + 255) / 256;
+        if (blocks <= 0x7FFFFFFF && ((uintptr_t)dense & 15) == 0) {
+            hipLaunchKernelGGL(pack_dense_columns, dim3((unsigned)blocks), dim3(256), 0, s, rhs, rhs_cs, (uint32_t)n,
+                               (uint32_t)k, (uint32_t)n_pad, (uint32_t)k_pad, dense);
+            return hipGetLastError();
+        }
+    }
     const dim3 grid((unsigned)(k_pad / 32), (unsigned)(n_pad / 32));
     hipLaunchKernelGGL(pack_dense_strided, grid, dim3(256), 0, s, rhs, rhs_rs, rhs_cs, (uint32_t)n, (uint32_t)k,
                        (uint32_t)k_pad, dense);

@@ -89,6 +89,13 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
                        const uint16_t *lhs, long lhs_cs, long lhs_rs, float beta,
                        const EpArgs &ep, bool bf16, hipStream_t s, bool read_dst = false,
                        float alpha = 0.0f);
+// launch_gemm of dense weights with A packed first into scratch
+// (dense_pack_a_bytes, 16-byte aligned; 0 where launch_gemm reads A as well as
+// it is).
+size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs);
+hipError_t launch_gemm_pack_a(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
+                              long lhs_cs, long lhs_rs, float beta, const EpArgs &ep, bool bf16, uint16_t *scratch,
+                              hipStream_t s, bool read_dst = false, float alpha = 0.0f);
 // Dense F16/BF16 weights ([n_pad][k_pad], column j's K contiguous, zero
 // padded) from a k x n matrix B[l][j] = rhs[l*rhs_rs + j*rhs_cs].
 hipError_t launch_pack_dense_strided(const uint16_t *rhs, long rhs_rs, long rhs_cs, size_t n, size_t k,

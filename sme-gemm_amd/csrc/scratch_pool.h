@@ -46,6 +46,15 @@ public:
         return nb;
     }
 
+    // The buffer (device, stream) already has, if it holds `bytes`; nullptr
+    // otherwise (nothing is allocated).
+    void *find(int device, const void *stream, size_t bytes) const {
+        std::lock_guard<std::mutex> lk(mu_);
+        for (const Entry &e : live_)
+            if (e.device == device && e.stream == stream) return e.cap >= bytes ? e.buf : nullptr;
+        return nullptr;
+    }
+
     size_t live_count() const { std::lock_guard<std::mutex> lk(mu_); return live_.size(); }
     size_t retired_count() const { std::lock_guard<std::mutex> lk(mu_); return retired_.size(); }
 

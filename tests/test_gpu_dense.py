@@ -114,3 +114,55 @@ def test_strided_result_may_share_memory_with_b(smg):
     want = a.double() @ b.double()
     smg.gemm_f16(m, n, k, bt, n, 1, a, k, 1, bt, 1, k, 0.0, 1.0)
     _check(bt, want, k, False)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("m,n,k", [(61, 499, 523), (1, 130, 7), (33, 65, 1), (300, 1001, 2049), (5, 9, 63)])
+def test_products_over_any_k(smg, m, n, k, bf16):
+    """K not a multiple of 8, unaligned rows and column strides: A packed on
+    the device (host, device, packed and strided calls alike), NaN outside
+    every view."""
+    import torch
+    a, b = _mats(m, n, k, bf16, m * k)
+    want = a.double() @ b.double()
+    p = (smg.prepack_bf16 if bf16 else smg.prepack_f16)(_bits(b), n, k)
+    mul = smg.matmul_bf16_packed if bf16 else smg.matmul_f16_packed
+    c = torch.empty(m, n, dtype=a.dtype, device="cuda")
+    mul(a, p, c, m)
+    _check(c, want, k, bf16)
+    ch = np.zeros(m * n, np.uint16)
+    mul(_bits(a).ravel(), p, ch, m)
+    assert np.array_equal(ch, _bits(c).ravel())
+    f = smg.gemm_bf16 if bf16 else smg.gemm_f16
+    at = torch.full((k, 2 * m + 1), float("nan"), dtype=a.dtype, device="cuda")
+    at[:, 1::2][:, :m] = a.t()  # A[i, l] at 1 + 2 i + l (2 m + 1)
+    bt = torch.full((n, k + 1), float("nan"), dtype=a.dtype, device="cuda")
+    bt[:, 1:] = b.t()
+    c0 = torch.randn(m, n, device="cuda").to(a.dtype)
+    c = c0.clone()
+    f(m, n, k, c, n, 1, at.view(-1)[1:], 2, 2 * m + 1, bt.view(-1)[1:], 1, k + 1, 0.5, 1.0)
+    _check(c, want + 0.5 * c0.double(), k, bf16)
+
+
+def test_odd_k_product_captured_without_scratch(smg):
+    """A first odd-K product on a stream under capture allocates nothing (it
+    reads A as it is) and replays right; eager calls on the stream then pack."""
+    import torch
+    m, n, k = 40, 200, 333
+    a, b = _mats(m, n, k, False, 5)
+    p = smg.prepack_f16(_bits(b), n, k)
+    c, e = (torch.empty(m, n, dtype=a.dtype, device="cuda") for _ in range(2))
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        smg.matmul_f16_packed(a, p, c, m)
+    for seed in (6, 7):
+        a.copy_(_mats(m, n, k, False, seed)[0])
+        g.replay()
+        torch.cuda.synchronize()
+        _check(c, a.double() @ b.double(), k, False)
+        with torch.cuda.stream(s):
+            smg.matmul_f16_packed(a, p, e, m)
+        torch.cuda.synchronize()
+        _check(e, a.double() @ b.double(), k, False)
