@@ -521,6 +521,8 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
     if (read_dst && w.kind != W_F16 && w.kind != W_BF16) return hipErrorInvalidValue;
     if (!read_dst && q4r_supported(w, m, lhs_cs, lhs_rs, lhs, bf16))
         return launch_q4r(w, m, dst, dst_cs, dst_rs, lhs, lhs_rs, beta, ep, nullptr, 0, bf16, s);
+    if (!read_dst && gemm_mopa_supported(w, m, lhs_cs, lhs_rs, lhs))
+        return launch_gemm_mopa(w, m, dst, dst_cs, dst_rs, lhs, lhs_rs, beta, ep, s);
     if (w.kind == W_F16 || w.kind == W_BF16) {
         const DenseGemm d = {lhs, w.dense, dst, m, w.n, w.k, w.n_pad, lhs_rs, (long)w.k_pad, dst_rs, dst_cs,
                              beta, alpha, read_dst};
@@ -712,7 +714,8 @@ hipError_t launch_q4_dequant_dense(const WDev &q4, uint16_t *dense, bool to_bf16
 }  // namespace smg
 
 // The DMA-staged GEMMs, part of this translation unit: launch_gemm's dense
-// kernels, and the low-bit int8 one, whose arguments are not preloaded as
+// and low-bit f16 kernels, and the low-bit int8 one, whose arguments are not preloaded as
 // lowbit_gemv.hip's are.
 #include "gemm_dense.cuh"
+#include "gemm_mopa.cuh"
 #include "lowbit_gemm.cuh"

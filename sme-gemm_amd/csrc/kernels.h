@@ -116,6 +116,12 @@ struct DenseGemm {
 bool gemm_dense_supported(const DenseGemm &d);
 hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hipStream_t s);
 
+// The f16 GEMM over low-bit weights (gemm_mopa.cuh); launch_gemm uses it
+// whenever gemm_mopa_supported holds.
+bool gemm_mopa_supported(const WDev &w, size_t m, long lhs_cs, long lhs_rs, const uint16_t *lhs);
+hipError_t launch_gemm_mopa(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
+                            long lhs_rs, float beta, const EpArgs &ep, hipStream_t s);
+
 // Q4 GEMM with register-resident weights (gemm_q4r.hip): f16 or bf16
 // activations, block >= 32, K a multiple of 64, row-major 16-byte-aligned A.
 // launch_gemm uses it whenever q4r_supported holds.
