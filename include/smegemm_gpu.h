@@ -267,7 +267,9 @@ int gemm_gpu_bf16f32_run(size_t m, size_t n, size_t k, uint16_t *dst, long dst_c
                          const uint16_t *rhs, long rhs_cs, long rhs_rs, uint16_t alpha_bits,
                          uint16_t beta_bits);
 /* The same on device pointers, enqueued on `stream` (bf16 != 0: bf16 operands);
- * B is packed into a scratch buffer of the stream's own (grow-only, kept). */
+ * a column-major, 16-byte-aligned B is read in place unless it overlaps C, any
+ * other is packed, as is an A of unaligned rows, into a scratch buffer of the
+ * stream's own (grow-only, kept). */
 int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long dst_cs, long dst_rs,
                      int read_dst, const uint16_t *lhs, long lhs_cs, long lhs_rs, const uint16_t *rhs,
                      long rhs_cs, long rhs_rs, uint16_t alpha_bits, uint16_t beta_bits, void *stream);
@@ -324,6 +326,9 @@ int smg_lowbit_matmul_dev_noalloc(size_t m, const smg_weights *w, uint16_t *dst,
                                   const uint16_t *lhs, const ep_desc16 *ep, void *stream);
 int smg_lowbit_mopa_dev(size_t m, const smg_weights *w, uint16_t *dst, const uint16_t *lhs,
                         const ep_desc16 *ep, void *stream);
+/* An A with K not a multiple of 8, unaligned rows or a column stride is packed
+ * into the stream's scratch first; while the stream is captured only into
+ * scratch that is there already, else the product reads A as it is. */
 int smg_packed_matmul_dev(size_t m, const smg_weights *b_pack, uint16_t *dst, long dst_cs,
                           long dst_rs, const uint16_t *lhs, long lhs_cs, long lhs_rs,
                           uint16_t beta_bits, const ep_desc16 *ep, int bf16, void *stream);

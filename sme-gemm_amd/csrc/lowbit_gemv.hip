@@ -11,7 +11,8 @@
 //      with the product scale*s rounded on its own;
 //   4. f16 RNE, then the op-graph.
 //
-// Two kernels per call:
+// Two kernels per call (from LOWBIT_GEMM_ROWS rows lowbit_gemm.cuh's, where it
+// takes the block size and its scratch can be had):
 // lowbit_quant: one workgroup per (row, block): q (int8), s and sum(q) into a
 //   small device buffer (the activations are read once, not once per column
 //   tile).
