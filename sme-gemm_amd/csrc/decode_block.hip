@@ -911,21 +911,28 @@ __global__ void __launch_bounds__(AP_T) attn_rows_mfma(AttnArgs a) {
 //   operand comes from the row-major values by the transposing LDS read
 //   (ds_read_b64_tr_b16: 4 keys x 16 depths a 16-lane group) with the same key
 //   order.
-// A row's running max only moves when a score passes it by more than 8 in
-// log2 (the probabilities stay below 2^8, as exact in f16 as below 1), so the
-// usual block has no cross-lane step and no rescale; the row sums stay per
+// The cross-lane maximum and the rescale run only in a block where a score
+// passes its row's running max, so a key quarter's largest probability is
+// exactly 1. (Letting the max lag until a probability would pass 2^8 takes 0 to
+// 10 us less but loses precision: the largest probability's own f16 rounding then
+// weighs most, and the row sum, of the unrounded values, does not share it. Error
+// against 64 bits, 512 rows after 4096 positions, 32 heads of 128 over 8, scores
+// of deviation 1 / 3 / 10: 2.05e-4 / 1.59e-4 / 8.7e-5 there, 1.83e-4 / 5.3e-5 /
+// 2.1e-5 here, 1.94e-4 / 8.0e-5 / 3.9e-5 in attn_rows_mfma.) The row sums stay per
 // lane until the end, where the four key quarters of a unit are merged through
 // LDS. Masks (scores, and values past the unit's last position, so that no
 // row's probability of zero meets them) only where a wave's keys reach the
 // unit's own positions.
-// What bounds it: about 130 vector instructions (16 of them 2^x) and 32 products
-// a wave and block, two waves a SIMD, one barrier a block. Measured (us, one
-// MI355X, q's rounding pass included; attn_rows_mfma, one wave a SIMD with 160
-// KB of LDS traffic a 64-key block, before): 512 rows after 4096 positions, 32
-// heads of 128 over 8 KV heads 136 -> 69, over 32 KV heads 373 -> 68; 1024 rows
-// after 8192 370 -> 226; 32 rows after 8192, 12 heads of 64, 145 -> 55. Kept out:
-// wave groups one phase apart with a barrier between scores and values (87),
-// both in lockstep phases (77): the barrier's wait exceeds what it overlaps.
+// What bounds it: the vector instructions (16 of them 2^x, and the rescale's 64
+// in most early blocks) and 32 products a wave and block, two waves a SIMD, one
+// barrier a block. Measured (us, one MI355X, q's rounding pass included;
+// attn_rows_mfma, one wave a SIMD with 160 KB of LDS traffic a 64-key block,
+// before): 512 rows after 4096 positions, 32 heads of 128 over 8 KV heads 128 ->
+// 67, over 32 KV heads 353 -> 71; 1024 rows after 8192 367 -> 221; 2048 rows, 16
+// heads of 128 over 8, 123 -> 63; 32 rows after 8192, 12 heads of 64, 144 -> 64.
+// Kept out: wave groups one phase apart with a barrier between scores and values,
+// or both in lockstep phases: each a quarter slower, the barrier's wait exceeds
+// what it overlaps.
 constexpr int AD_T = 512, AD_KB = 128, AD_U = 4;  // threads, keys a block, units
 constexpr float AD_LOW = -1e30f;                  // below every finite score
 
@@ -944,6 +951,14 @@ struct AttnDma {
     static __device__ __forceinline__ uint32_t vsw(uint32_t r) { return HDM == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); }
 };
 
+// The maximum of a row's values in lanes l, l ^ 16, l ^ 32 and l ^ 48.
+__device__ __forceinline__ float four_lanes_max(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
 template <int HDM>
 __global__ void __launch_bounds__(AD_T) attn_rows_dma(AttnArgs a, uint32_t hg) {
     using T = AttnDma<HDM>;
@@ -959,9 +974,9 @@ __global__ void __launch_bounds__(AD_T) attn_rows_dma(AttnArgs a, uint32_t hg) {
     const uint32_t nkeys = a.len + min((tile0 + tiles) * 16, a.rows) - 1;  // the last position's prefix
     const uint32_t nblk = (nkeys + AD_KB - 1) / AD_KB;
 
-    // the wave's units: head, this lane's row, the first row's keys (fewer need
-    // no mask) and the last row's (0: no rows)
-    uint32_t head[2], row[2], first[2], ukeys[2];
+    // the wave's units: head, this lane's row and the last row's keys (0: no
+    // rows)
+    uint32_t head[2], row[2], ukeys[2];
     u32x4_t qf[2][KK];
     const rsrc_t qr = make_rsrc(a.q, a.rows * a.heads * a.hd * 2u);
 #pragma unroll
@@ -969,7 +984,6 @@ __global__ void __launch_bounds__(AD_T) attn_rows_dma(AttnArgs a, uint32_t hg) {
         const uint32_t u = 2 * up + j, p0 = (tile0 + u / hg) * 16;
         head[j] = kvh * a.group + hc0 + u % hg;
         row[j] = p0 + r16;
-        first[j] = a.len + p0;
         ukeys[j] = p0 < a.rows ? a.len + min(p0 + 16, a.rows) - 1 : 0;
 #pragma unroll
         for (int kk = 0; kk < KK; kk++) {
@@ -1056,18 +1070,21 @@ __global__ void __launch_bounds__(AD_T) attn_rows_dma(AttnArgs a, uint32_t hg) {
 #pragma unroll
             for (int e = 1; e < 8; e++) mx[j] = fmaxf(mx[j], sc[j][e / 4][e % 4]);
         }
-        const float over = fmaxf(__builtin_fmaf(mx[0], LOG2E, -m2[0]), __builtin_fmaf(mx[1], LOG2E, -m2[1]));
-        if (__builtin_amdgcn_ballot_w64(over > 8.0f) != 0) {
-            // some row's max moved: the rows' new max over their four lanes
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                mx[j] = fmaxf(mx[j], xor_lanes(mx[j], 16));
-                mx[j] = fmaxf(mx[j], xor_lanes(mx[j], 32));
-                const float mn = fmaxf(m2[j], mx[j] * LOG2E);
+        for (int j = 0; j < 2; j++) {
+            // (the product rounds as it did when it became m2: the same maximum
+            // does not move it again)
+            if (__builtin_amdgcn_ballot_w64(mx[j] * LOG2E > m2[j]) != 0) {
+                // some row's max moved: the rows' new max over their four lanes
+                const float mn = fmaxf(m2[j], four_lanes_max(mx[j]) * LOG2E);
                 const float alpha = m2[j] == mn ? 1.0f : __builtin_amdgcn_exp2f(m2[j] - mn);
                 m2[j] = mn;
                 l[j] = l[j] * alpha;
-                // (in place: otherwise the merge of the two paths copies every o)
+                // (in place: otherwise the merge of the two paths copies every o.
+                // The compiler does not count the products' latency, 12 issue slots,
+                // against inline asm: the ten instructions up to alpha and these
+                // four cover it.)
+                asm volatile("s_nop 3");
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++)
 #pragma unroll

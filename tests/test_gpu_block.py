@@ -898,3 +898,35 @@ def test_causal_rows_dma_keeps_later_positions_out(smg):
     smg.attention_kv_causal_f16(q, k, v, start, rows, heads, heads, hd, hd ** -0.5, out)
     assert bool(torch.isfinite(out[:48]).all())
     assert bool(out[50:].isnan().all())
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,start,rows", [(8, 2, 128, 1000, 64), (4, 4, 64, 2000, 96),
+                                                          (4, 2, 80, 0, 300)])
+@pytest.mark.parametrize("dev", [1.0, 3.0, 10.0])
+def test_causal_rows_dma_error_is_no_larger(smg, heads, kv_heads, hd, start, rows, dev):
+    """The DMA-staged form's error against 64 bits is no larger than
+    attn_rows_mfma's on the same inputs, for scores of deviations 1 (flat rows)
+    to 10 (peaked ones). Both round probabilities to f16 against the row's own
+    maximum, whose probability is exactly 1; an out that is not 16-byte aligned
+    takes attn_rows_mfma."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(int(dev) * 100 + hd)
+    ln, ql, ld = start + rows, heads * hd, kv_heads * hd
+    q = torch.randn(rows, ql, generator=g, device="cuda") * dev
+    k, v = (torch.randn(ln, ld, generator=g, device="cuda").half() for _ in range(2))
+    scale = hd ** -0.5
+    dma = torch.empty(rows * ql, device="cuda")
+    mfma = torch.empty(rows * ql + 1, device="cuda")[1:]
+    assert dma.data_ptr() % 16 == 0 and mfma.data_ptr() % 16 == 4
+    for out in (dma, mfma):
+        smg.attention_kv_causal_f16(q, k, v, start, rows, heads, kv_heads, hd, scale, out)
+    qs = (q * scale).half().double()
+    mask = torch.arange(ln, device="cuda")[None] > start + torch.arange(rows, device="cuda")[:, None]
+    want = torch.empty(rows, ql, dtype=torch.float64, device="cuda")
+    for h in range(heads):
+        j = h // (heads // kv_heads)
+        s = qs[:, h * hd:(h + 1) * hd] @ k[:, j * hd:(j + 1) * hd].double().t().contiguous()
+        want[:, h * hd:(h + 1) * hd] = (torch.softmax(s.masked_fill(mask, -float("inf")), 1)
+                                        @ v[:, j * hd:(j + 1) * hd].double().contiguous())
+    err = [(x.double().view(rows, ql) - want).norm().item() for x in (dma, mfma)]
+    assert err[0] <= err[1], err
