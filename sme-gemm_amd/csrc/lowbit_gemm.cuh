@@ -388,10 +388,11 @@ hipError_t launch_lg_rows(const LgArgs &g, const EpArgs &ep, int epv, hipStream_
 
 size_t lowbit_gemm_bytes(const WDev &w, size_t m) {
     if (m < LOWBIT_GEMM_ROWS || w.k == 0 || w.n == 0 || (w.block != 64 && w.block != 128 && w.block != 256)) return 0;
-    // the GEMV's limits: a buffer resource spans < 2 GiB
+    // the GEMV's limits (a buffer resource spans < 2 GiB), and a column's code
+    // offset, 256 bytes of stride a column, in the DMA's 32-bit lane offset
     const size_t kq = (w.k + w.block - 1) / w.block * w.block;
     if (m * kq >= ((size_t)1 << 31) || m * w.k * 2 >= ((size_t)1 << 31) ||
-        cell_grid_rows(w.sc_rows) * w.n_pad * 2 >= ((size_t)1 << 31))
+        cell_grid_rows(w.sc_rows) * w.n_pad * 2 >= ((size_t)1 << 31) || w.n_pad * 256 >= ((size_t)1 << 31))
         return 0;
     const size_t blocks = lg_steps(w) * (LG_STEP / w.block);
     return lg_q_bytes(w, m) + blocks * ((m + 15) / 16 * 16) * sizeof(float);

@@ -1,0 +1,52 @@
+// The dispatch rules' bounds on sizes whose arrays need not exist: only host
+// code of the launch interface runs, nothing reaches a GPU.
+#include <cstdio>
+
+#include "kernels.h"
+
+using namespace smg;
+
+static int failed = 0;
+#define CHECK(c)                                                  \
+    do {                                                          \
+        if (!(c)) {                                               \
+            std::printf("line %d: %s does not hold\n", __LINE__, #c); \
+            failed++;                                             \
+        }                                                         \
+    } while (0)
+
+static WDev lowbit(int kind, size_t n, size_t k, size_t block) {
+    const size_t group = kind == W_Q2 ? Q2_GROUP : Q1_GROUP;
+    WDev w = {};
+    w.kind = kind;
+    w.n = n;
+    w.k = k;
+    w.block = block;
+    w.n_pad = (n + 127) / 128 * 128;
+    w.nchunks = (k + group - 1) / group;
+    w.sc_rows = (k + block - 1) / block;
+    return w;
+}
+
+// Byte offset of the last column's codes from the first's, as a GEMM lane
+// adds it to its step's base.
+static size_t last_code(const WDev &w) { return cell_col_part(w.n_pad - 1, 0, w.n_pad) * 64 + 3 * 16 + 16; }
+
+int main() {
+    const int kinds[2] = {W_Q2, W_Q1};
+    // The many-row GEMM serves a call only where a column's code offset fits the
+    // DMA's 32-bit lane offset.
+    for (int kind : kinds)
+        for (size_t block : {(size_t)64, (size_t)128, (size_t)256})
+            for (size_t n : {(size_t)1, (size_t)11008, ((size_t)1 << 23) - 128, (size_t)1 << 23, ((size_t)1 << 24) - 1,
+                             (size_t)1 << 24, ((size_t)1 << 24) + 1, (size_t)1 << 25, (size_t)1 << 27}) {
+                const WDev w = lowbit(kind, n, 64, block);
+                const size_t bytes = lowbit_gemm_bytes(w, 9);
+                CHECK(bytes == 0 || last_code(w) <= 0xFFFFFFFFu);
+                CHECK(n >= ((size_t)1 << 23) || bytes != 0);  // ordinary widths stay on it
+                const uint16_t *a = (const uint16_t *)256;
+                CHECK(!gemm_mopa_supported(w, 512, 1, 64, a) || last_code(w) <= 0xFFFFFFFFu);
+            }
+    if (failed == 0) std::printf("dispatch rules ok\n");
+    return failed != 0;
+}

@@ -83,3 +83,28 @@ def test_library_host_code_under_asan(tmp_path):
                UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120, env=env)
     assert r.returncode == 0 and "host asan ok" in r.stdout, r.stdout + r.stderr
+
+
+def _library_objects():
+    """The library's objects, built if any is missing."""
+    pkg = os.path.join(ROOT, "sme-gemm_amd")
+    names = [f[:-4] for f in sorted(os.listdir(os.path.join(pkg, "csrc"))) if f.endswith(".hip")]
+    objs = [os.path.join(pkg, "_build", f + ".o") for f in names]
+    if not all(os.path.exists(o) for o in objs):
+        subprocess.run(["make", "-s", "-j8", "-C", pkg], check=True, timeout=900)
+    return objs
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+def test_dispatch_rules(tmp_path):
+    """The launch interface's rules (csrc/kernels.h) at the edges of their ranges,
+    on the host alone."""
+    drv, exe = str(tmp_path / "drv.o"), str(tmp_path / "dispatch_rules_test")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O1", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-I", os.path.join(ROOT, "sme-gemm_amd", "csrc"), "-x", "hip", "-c",
+                    os.path.join(CPP, "dispatch_rules_test.cpp"), "-o", drv], check=True, timeout=300,
+                   capture_output=True)
+    subprocess.run([HIPCC, "--offload-arch=gfx950", *_library_objects(), drv, "-o", exe, "-lpthread"], check=True,
+                   timeout=300, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "dispatch rules ok" in r.stdout, r.stdout + r.stderr
