@@ -327,8 +327,10 @@ int smg_lowbit_matmul_dev_noalloc(size_t m, const smg_weights *w, uint16_t *dst,
 int smg_lowbit_mopa_dev(size_t m, const smg_weights *w, uint16_t *dst, const uint16_t *lhs,
                         const ep_desc16 *ep, void *stream);
 /* An A with K not a multiple of 8, unaligned rows or a column stride is packed
- * into the stream's scratch first; while the stream is captured only into
- * scratch that is there already, else the product reads A as it is. */
+ * first, into scratch that the call holds for its two launches (calls of several
+ * host threads on one stream stay apart). While the stream is captured, and
+ * where no scratch can be had, the product reads A as it is: a graph holds no
+ * scratch of this call. */
 int smg_packed_matmul_dev(size_t m, const smg_weights *b_pack, uint16_t *dst, long dst_cs,
                           long dst_rs, const uint16_t *lhs, long lhs_cs, long lhs_rs,
                           uint16_t beta_bits, const ep_desc16 *ep, int bf16, void *stream);

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "kernels.h"
+#include "lease_pool.h"
 #include "scratch_pool.h"
 
 using namespace smg;
@@ -120,6 +121,16 @@ int ctx_for(int device, size_t bytes, Ctx **out) {
     return SMG_OK;
 }
 
+// Whether the stream is being captured into a graph (then no call allocates).
+bool stream_capturing(void *stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;  // (the null stream beside another one's capture)
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // ---- device-pointer scratch ---------------------------------------------------
 // The *_dev entry points return before their kernels run, and a HIP graph may
 // replay those kernels later still, so their scratch is never the thread's
@@ -140,6 +151,45 @@ struct HipDevAlloc {
 ScratchPool<HipDevAlloc> &dev_pool() {
     static ScratchPool<HipDevAlloc> *p = new ScratchPool<HipDevAlloc>();  // never destroyed
     return *p;
+}
+
+// ---- the packed product's A -----------------------------------------------------
+// smg_packed_matmul_dev's copy of an A that the dense tiles cannot read: two
+// launches meet in it, in a call that has no other scratch, so it is leased for
+// both of them (lease_pool.h) and no graph holds it. (A new stream may get a
+// destroyed one's handle, and with it the buffer: hipStreamDestroy has waited for
+// the work by then.)
+struct PackAlloc {
+    // Allocating or freeing is an error in a thread of the default capture mode
+    // while any stream is captured, and ends that capture; no stream that this
+    // memory is used on is.
+    struct Relaxed {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    };
+    void *acquire(int device, size_t bytes) {
+        Relaxed r;
+        void *p = HipDevAlloc().acquire(device, bytes);
+        if (!p) (void)hipGetLastError();
+        return p;
+    }
+    void release(int, void *p) {
+        Relaxed r;
+        (void)hipFree(p);
+    }
+};
+typedef LeasePool<PackAlloc> PackPool;
+// An empty lease where the stream is captured, or is each thread's own under one
+// handle.
+PackPool::Lease pack_lease(int device, void *stream, size_t bytes) {
+    static PackPool *pool = new PackPool(32, (size_t)4 << 30);  // never destroyed
+    if (stream == (void *)hipStreamPerThread || stream_capturing(stream)) return PackPool::Lease();
+    try {
+        return pool->take(device, stream, bytes);
+    } catch (...) {  // no host memory for its entry
+        return PackPool::Lease();
+    }
 }
 
 // ---- allocation-free scratch (smg_lowbit_matmul_dev_noalloc) --------------------
@@ -461,16 +511,6 @@ int make_dense(int kind, const uint16_t *rhs, size_t n, size_t k, long rs, long 
     d.dense = (const uint16_t *)p;
     *out = w;
     return SMG_OK;
-}
-
-// Whether the stream is being captured into a graph (then no call allocates).
-bool stream_capturing(void *stream) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return st != hipStreamCaptureStatusNone;
 }
 
 // ---- one host-pointer call ---------------------------------------------------
@@ -1794,17 +1834,15 @@ int smg_packed_matmul_dev(size_t m, const smg_weights *b, uint16_t *dst, long ds
     EpPlan ep_p;
     if ((rc = ep_plan(ep, &ep_p, b->d.n))) return rc;
     if ((rc = check_dev_ptrs("smg_packed_matmul_dev", b->device, stream, ep_p, {dst, lhs}))) return rc;
-    // A packed into the stream's scratch where gemm_dense cannot read it; without
-    // the scratch (none to be had, or none yet while the stream is captured)
-    // the product reads A as it is
+    // A packed first where gemm_dense cannot read it; without scratch for that
+    // (none to be had, or the stream is captured) the product reads A as it is
     const float beta = half_bits_to_float(beta_bits, bf16 != 0);
     const size_t ab = dense_pack_a_bytes(b->d, m, lhs, lhs_cs, lhs_rs);
-    void *ap = nullptr;
-    if (ab) ap = stream_capturing(stream) ? dev_pool().find(b->device, stream, ab) : dev_pool().get(b->device, stream, ab);
-    hipError_t e = ap ? launch_gemm_pack_a(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
-                                           (uint16_t *)ap, (hipStream_t)stream)
-                      : launch_gemm(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
-                                    (hipStream_t)stream);
+    const PackPool::Lease ap = ab ? pack_lease(b->device, stream, ab) : PackPool::Lease();
+    hipError_t e = ap.buf() ? launch_gemm_pack_a(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
+                                                 (uint16_t *)ap.buf(), (hipStream_t)stream)
+                            : launch_gemm(b->d, m, dst, dst_cs, dst_rs, lhs, lhs_cs, lhs_rs, beta, ep_p.fused, bf16 != 0,
+                                          (hipStream_t)stream);
     if (e == hipSuccess) e = plan_tail(ep_p, dst, dst_cs, dst_rs, m, b->d.n, bf16 != 0, (hipStream_t)stream);
     return e == hipSuccess ? SMG_OK : fail(SMG_EHIP, "smg_packed_matmul_dev", e);
 }

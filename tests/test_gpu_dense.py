@@ -166,3 +166,116 @@ def test_odd_k_product_captured_without_scratch(smg):
             smg.matmul_f16_packed(a, p, e, m)
         torch.cuda.synchronize()
         _check(e, a.double() @ b.double(), k, False)
+
+
+def test_odd_k_graphs_hold_no_scratch(smg):
+    """Two graphs captured on one stream after eager calls warmed it, replayed on
+    two streams at once beside eager calls on the capture stream: each reads its
+    own A (a packed copy in the stream's scratch would be overwritten by the
+    others)."""
+    import torch
+    m, n, k = 1000, 500, 1001
+    b = _mats(m, n, k, False, 5)[1]
+    p = smg.prepack_f16(_bits(b), n, k)
+    cap = torch.cuda.Stream()
+    a = [_mats(m, n, k, False, 20 + i)[0] for i in range(3)]
+    c = [torch.empty(m, n, dtype=torch.float16, device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(cap):
+        smg.matmul_f16_packed(a[2], p, c[2], m)  # scratch of the largest size is there
+    torch.cuda.synchronize()
+    graphs = []
+    for i in range(2):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cap):
+            for _ in range(4):
+                smg.matmul_f16_packed(a[i], p, c[i], m)
+        graphs.append(g)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for rep in range(4):
+        for i in range(3):
+            a[i].copy_(_mats(m, n, k, False, 100 * rep + i)[0])
+            c[i].fill_(float("nan"))
+        torch.cuda.synchronize()
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                graphs[i].replay()
+        with torch.cuda.stream(cap):
+            for _ in range(4):
+                smg.matmul_f16_packed(a[2], p, c[2], m)
+        torch.cuda.synchronize()
+        for i in range(3):
+            _check(c[i], a[i].double() @ b.double(), k, False)
+
+
+def test_odd_k_calls_of_several_threads_on_one_stream(smg):
+    """Host threads that share a stream: a call's packing and product stay
+    together, whatever the threads' sizes (the scratch grows between them)."""
+    import threading
+    import torch
+    s = torch.cuda.Stream()
+    jobs, err = [], []
+    for t in range(4):
+        m, n, k = 400 + 300 * t, 200, 1001 + 2 * t
+        a, b = _mats(m, n, k, False, 60 + t)
+        p = smg.prepack_f16(_bits(b), n, k)
+        jobs.append((a, b, p, [torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda") for _ in range(24)]))
+    torch.cuda.synchronize()
+
+    def work(a, p, cs):
+        try:
+            with torch.cuda.stream(s):
+                for c in cs:
+                    smg.matmul_f16_packed(a, p, c, a.shape[0])
+        except Exception as e:  # noqa: BLE001
+            err.append(e)
+
+    ts = [threading.Thread(target=work, args=(a, p, cs)) for a, b, p, cs in jobs]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    torch.cuda.synchronize()
+    assert not err, err
+    for a, b, p, cs in jobs:
+        want = a.double() @ b.double()
+        for c in cs:
+            _check(c, want, a.shape[1], False)
+
+
+def test_odd_k_call_beside_another_threads_capture(smg):
+    """An eager call that needs scratch for the first time on its stream, while
+    this thread captures another stream in the default mode: neither the capture
+    nor the call fails."""
+    import threading
+    import torch
+    m, n, k = 2000, 96, 1003
+    a, b = _mats(m, n, k, False, 70)
+    p = smg.prepack_f16(_bits(b), n, k)
+    other, cap = torch.cuda.Stream(), torch.cuda.Stream()
+    c, d = (torch.empty(m, n, dtype=torch.float16, device="cuda") for _ in range(2))
+    smg.matmul_f16_packed(a[:16].contiguous(), p, c[:16].contiguous(), 16)  # kernels are loaded
+    torch.cuda.synchronize()
+    err = []
+
+    def call():
+        try:
+            with torch.cuda.stream(other):
+                smg.matmul_f16_packed(a, p, c, m)
+        except Exception as e:  # noqa: BLE001
+            err.append(e)
+
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        smg.matmul_f16_packed(a, p, d, m)
+        t = threading.Thread(target=call)
+        t.start()
+        t.join()
+    assert not err, err
+    want = a.double() @ b.double()
+    for _ in range(2):
+        d.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        _check(d, want, k, False)
+    _check(c, want, k, False)

@@ -36,6 +36,15 @@ def test_scratch_pool_growth_rule_under_asan(tmp_path):
     assert "scratch pool ok" in _run(exe)
 
 
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_lease_pool_under_asan(tmp_path):
+    """One holder a stream, bounds kept, buffers given back (csrc/lease_pool.h)."""
+    exe = str(tmp_path / "lease_pool_test")
+    subprocess.run(["g++", "-std=c++17", *SAN, "-pthread", os.path.join(CPP, "lease_pool_test.cpp"), "-o", exe],
+                   check=True, timeout=300)
+    assert "lease pool ok" in _run(exe)
+
+
 @pytest.mark.skipif(shutil.which("gcc") is None, reason="needs gcc")
 def test_oracle_under_asan(tmp_path):
     """Every oracle function on ragged shapes with exactly-sized buffers
