@@ -572,8 +572,11 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
 // of 8, rows not 16-byte aligned, a column stride): A is packed as B is, K zero
 // padded to B's k_pad, and the product runs over k_pad. gemm_kernel reads such
 // an A element by element. Measured with a prepacked B (us, the packing of A
-// included): 3000 x 500 x 3001 173 -> 41, 61 x 499 x 523 28 -> 7.8, one row x 4096
-// x 4097 122 -> 18.
+// included): 3000 x 500 x 3001 173 -> 41, 61 x 499 x 523 28 -> 11, one row x 4096
+// x 4097 122 -> 18. An A that only K < 64 keeps off the tiles it reads by
+// vectors, and the packing's launch costs more than it gains while gemm_kernel's
+// 256 x 128 tiles fit the compute units once: 16 x 500 x 8 7.7 read, 9.3 packed,
+// 2000 x 3000 x 32 10.8 and 12.1, 3000 x 3000 x 32 18.7 and 15.5.
 size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs) {
     if ((w.kind != W_F16 && w.kind != W_BF16) || m == 0 || w.n == 0 || w.k == 0 || lhs_cs < 0 || lhs_rs < 0) return 0;
     const size_t big = (size_t)1 << 31;
@@ -581,6 +584,9 @@ size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs
     if (fp >= big || rows * w.k_pad * 2 >= big || rows / 32 > 65535) return 0;
     const DenseGemm d = {lhs, w.dense, nullptr, m, w.n, w.k, w.n_pad, lhs_rs, (long)w.k_pad, 1, 1, 1.0f, 0.0f, false};
     if (lhs_cs == 1 && gemm_dense_supported(d)) return 0;
+    if (w.k < 64 && w.k % 8 == 0 && lhs_cs == 1 && lhs_rs % 8 == 0 && ((uintptr_t)lhs & 15) == 0 &&
+        ((m + 255) / 256) * ((w.n + 127) / 128) <= (size_t)device_cus())
+        return 0;
     return rows * w.k_pad * 2;
 }
 hipError_t launch_gemm_pack_a(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,

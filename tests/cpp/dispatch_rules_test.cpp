@@ -47,6 +47,27 @@ int main() {
                 const uint16_t *a = (const uint16_t *)256;
                 CHECK(!gemm_mopa_supported(w, 512, 1, 64, a) || last_code(w) <= 0xFFFFFFFFu);
             }
+
+    // Dense products: an A is packed where the tiles cannot read it and packing
+    // pays. K < 64 alone is no reason (gemm_kernel reads such rows by vectors)
+    // until gemm_kernel's own tiles need a second round.
+    for (size_t k : {(size_t)1, (size_t)8, (size_t)31, (size_t)32, (size_t)56, (size_t)63, (size_t)64, (size_t)72,
+                     (size_t)1001})
+        for (size_t m : {(size_t)1, (size_t)16, (size_t)500, (size_t)3000})
+            for (size_t n : {(size_t)100, (size_t)500, (size_t)3000}) {
+                WDev w = {};
+                w.kind = W_F16;
+                w.n = n;
+                w.k = k;
+                w.n_pad = (n + 127) / 128 * 128;
+                w.k_pad = (k + 63) / 64 * 64;
+                w.dense = (const uint16_t *)4096;
+                const uint16_t *a = (const uint16_t *)256;
+                const bool vec = k % 8 == 0, two = m * n >= (size_t)9000000;
+                CHECK((dense_pack_a_bytes(w, m, a, 1, (long)k) != 0) == (!vec || (k < 64 && two)));
+                CHECK(dense_pack_a_bytes(w, m, a + 1, 1, (long)k) != 0);         // unaligned rows
+                CHECK(dense_pack_a_bytes(w, m, a, (long)m, 1) != 0 || (m == 1 && k == 1));  // a column stride
+            }
     if (failed == 0) std::printf("dispatch rules ok\n");
     return failed != 0;
 }
