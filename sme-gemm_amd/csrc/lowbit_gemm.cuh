@@ -386,8 +386,22 @@ hipError_t launch_lg_rows(const LgArgs &g, const EpArgs &ep, int epv, hipStream_
 
 }  // namespace
 
+// Calls the 16-row GEMV takes no longer than the GEMM: blocks of 256 (a GEMV
+// wave's own products of a block, and a fold a 256-depth step here) past 2048
+// depths, few rows, and GEMV workgroups (16 rows x 16 columns) that fit the
+// compute units once, so that no weight is waited for twice. 2-bit, us, GEMV and
+// GEMM: 9 rows x 700 x 8000 16.0 / 18.8, 32 x 2048 x 4096 12.2 / 12.5, 48 x 700 x
+// 4096 12.3 / 13.0; the other side: 33 x 2048 x 8000 20.8 / 18.6 (a second round),
+// 64 x 128 x 16000 33.5 / 31.1 (a row group's loads compete for longer), 9 x 700 x
+// 2048 10.1 / 10.3, blocks of 128 9 x 2048 x 8000 18.5 / 18.1.
+static bool lowbit_gemv_faster(const WDev &w, size_t m) {
+    constexpr size_t CUS = 256;  // (a constant: scratch is sized by the same rule, on any current device)
+    return w.block == 256 && w.k > 2048 && m <= (w.k <= 8192 ? 64 : 32) && (m + 15) / 16 * (w.n_pad / 16) <= CUS;
+}
+
 size_t lowbit_gemm_bytes(const WDev &w, size_t m) {
     if (m < LOWBIT_GEMM_ROWS || w.k == 0 || w.n == 0 || (w.block != 64 && w.block != 128 && w.block != 256)) return 0;
+    if (lowbit_gemv_faster(w, m)) return 0;
     // the GEMV's limits (a buffer resource spans < 2 GiB), and a column's code
     // offset, 256 bytes of stride a column, in the DMA's 32-bit lane offset
     const size_t kq = (w.k + w.block - 1) / w.block * w.block;

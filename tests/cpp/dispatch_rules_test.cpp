@@ -48,6 +48,18 @@ int main() {
                 CHECK(!gemm_mopa_supported(w, 512, 1, 64, a) || last_code(w) <= 0xFFFFFFFFu);
             }
 
+    // Blocks of 256, past 2048 depths, few rows, one round of GEMV workgroups: the
+    // GEMV; each limit by one step on either side.
+    for (int kind : kinds) {
+        const size_t calls[][4] = {{9, 700, 8000, 1},   {9, 700, 2048, 0},   {9, 700, 2049, 1},   {32, 2048, 4096, 1},
+                                   {33, 2048, 4096, 0}, {16, 4096, 4096, 1}, {16, 4097, 4096, 0}, {64, 1024, 8192, 1},
+                                   {65, 128, 8192, 0},  {33, 128, 8193, 0},  {32, 128, 8193, 1}};
+        for (const auto &c : calls) {
+            CHECK((lowbit_gemm_bytes(lowbit(kind, c[1], c[2], 256), c[0]) == 0) == (c[3] != 0));
+            CHECK(lowbit_gemm_bytes(lowbit(kind, c[1], c[2], 128), c[0]) != 0);
+            CHECK(lowbit_gemm_bytes(lowbit(kind, c[1], c[2], 64), c[0]) != 0);
+        }
+    }
     // Dense products: an A is packed where the tiles cannot read it and packing
     // pays. K < 64 alone is no reason (gemm_kernel reads such rows by vectors)
     // until gemm_kernel's own tiles need a second round.
