@@ -1404,6 +1404,19 @@ size_t attn_partial_floats(size_t rows, size_t last_len, size_t heads, size_t hd
 
 bool attn_rows_blocked(size_t rows) { return rows >= AP_MIN_ROWS; }
 
+// Whether attn_rows_dma takes the rows: what it can address, and not the few
+// short rows of a wide head that attn_rows_mfma has done before its tiles are
+// there (us, attn_rows_mfma and attn_rows_dma, 64 rows: 16 heads of 128 over 8, 64
+// keys 10.8 / 11.9, 163 keys 13.0 / 14.1; 8 of 80 over 2, 191 keys 12.5 / 13.6; 32
+// of 128 over 8, 163 keys 15.0 / 14.6; the other side: 32 of 128 over 8, 363 keys
+// 19.8 / 16.4, 100 rows and keys 13.0 / 12.6; 12 of 64, 64 keys, 11.3 / 11.3).
+bool attn_rows_staged(const AttnArgs &a) {
+    const size_t last = (size_t)a.len + a.rows - 1;
+    if (a.hd > 64 && a.rows <= 64 && last <= 192) return false;
+    return a.hd <= 128 && (last + AD_KB) * a.ld * 2 < ((size_t)1 << 31) && a.ld % 8 == 0 &&
+           (((uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.q | (uintptr_t)a.out) & 15) == 0;
+}
+
 hipError_t launch_attention(const AttnArgs &a0, void *out, bool f16_out, hipStream_t s) {
     AttnArgs a = a0;
     if (a.rows == 0) a.rows = 1;
@@ -1418,8 +1431,7 @@ hipError_t launch_attention(const AttnArgs &a0, void *out, bool f16_out, hipStre
         if ((size_t)a.rows * a.heads * a.hd * 2 >= ((size_t)1 << 31)) return hipErrorInvalidValue;
         a.out = out;
         a.f16_out = f16_out ? 1u : 0u;
-        if (a.hd <= 128 && (last + AD_KB) * a.ld * 2 < ((size_t)1 << 31) && a.ld % 8 == 0 &&
-            (((uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.q | (uintptr_t)a.out) & 15) == 0) {
+        if (attn_rows_staged(a)) {
             const uint32_t hg = a.group % 4 == 0 ? 4 : a.group % 2 == 0 ? 2 : 1, tr = 16 * AD_U / hg;
             const dim3 dgrid(((a.rows + tr - 1) / tr) * (a.heads / hg));
             if (a.hd <= 64) hipLaunchKernelGGL(attn_rows_dma<64>, dgrid, dim3(AD_T), 0, s, a, hg);

@@ -210,6 +210,8 @@ size_t attn_splits(size_t len);
 // Partial-sum bytes (po, then pml) launch_attention needs for `rows` rows whose
 // last attends to `last_len` keys.
 size_t attn_partial_floats(size_t rows, size_t last_len, size_t heads, size_t hd);
+// Whether a block of rows (AttnArgs::out set) runs on the form staged by DMA.
+bool attn_rows_staged(const AttnArgs &a);
 hipError_t launch_attention(const AttnArgs &a, void *out, bool f16_out, hipStream_t s);
 // m rows of a qkv projection's f16 output (the device column order of the
 // fused QKV store) to attention inputs at positions pos0 .. pos0 + m - 1:

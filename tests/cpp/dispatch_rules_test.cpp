@@ -80,6 +80,29 @@ int main() {
                 CHECK(dense_pack_a_bytes(w, m, a + 1, 1, (long)k) != 0);         // unaligned rows
                 CHECK(dense_pack_a_bytes(w, m, a, (long)m, 1) != 0 || (m == 1 && k == 1));  // a column stride
             }
+    // Attention of row blocks: few short rows of a wide head stay on
+    // attn_rows_mfma, as does what attn_rows_dma cannot address.
+    {
+        const struct {
+            uint32_t heads, kv, hd, start, rows, staged;
+        } calls[] = {{16, 8, 128, 0, 64, 0},  {16, 8, 128, 128, 64, 0}, {16, 8, 128, 129, 64, 1}, {16, 8, 128, 0, 65, 1},
+                     {32, 8, 128, 160, 32, 0}, {32, 8, 128, 161, 32, 1}, {12, 12, 64, 0, 32, 1},  {12, 12, 72, 0, 32, 0},
+                     {4, 4, 256, 4096, 512, 0}, {32, 8, 128, 4096, 512, 1}, {6, 1, 128, 0, 32, 0}};
+        for (const auto &c : calls) {
+            AttnArgs a = {};
+            a.q = a.k = a.v = (const uint16_t *)256;
+            a.out = (void *)512;
+            a.heads = c.heads;
+            a.group = c.heads / c.kv;
+            a.hd = c.hd;
+            a.ld = c.kv * c.hd;
+            a.len = c.start + 1;
+            a.rows = c.rows;
+            CHECK(attn_rows_staged(a) == (c.staged != 0));
+            a.out = (void *)516;
+            CHECK(!attn_rows_staged(a));
+        }
+    }
     if (failed == 0) std::printf("dispatch rules ok\n");
     return failed != 0;
 }

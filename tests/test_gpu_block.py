@@ -860,7 +860,8 @@ def test_layer_norm_block_gpt2_style(smg, orc, rows, bias):
 # tile, key blocks of 128 whose last one is short, padded head dims, prefixes
 # that end on and beside a block.
 @pytest.mark.parametrize("heads,kv_heads,hd,start,rows", [
-    (8, 2, 128, 96, 32), (8, 2, 128, 97, 33), (4, 2, 64, 0, 70), (6, 2, 80, 300, 47), (3, 3, 64, 1, 65),
+    (8, 2, 128, 96, 32), (8, 2, 128, 97, 33), (8, 2, 128, 224, 32), (8, 2, 128, 224, 33), (4, 2, 64, 0, 70),
+    (6, 2, 80, 300, 47), (3, 3, 64, 1, 65),
     (5, 5, 128, 127, 129), (12, 1, 8, 128, 40), (2, 1, 16, 255, 64), (4, 4, 120, 500, 31 + 64)])
 def test_causal_rows_dma_tiles(smg, heads, kv_heads, hd, start, rows):
     """Against float64 softmax attention on the f16-rounded q * scale, whose
