@@ -420,6 +420,11 @@ hipError_t launch_dense_shape(const DArgs &g, const EpArgs &ep, int epv, hipStre
 
 }  // namespace
 
+TileDims gemm_dense_tile_dims(size_t m, size_t n, size_t k) {
+    const DCost &c = DENSE_TILES[dense_pick(m, n, k)];
+    return {c.bm, c.bn};
+}
+
 bool gemm_dense_supported(const DenseGemm &d) {
     const size_t big = (size_t)1 << 31;
     return d.m > 0 && d.n > 0 && d.k >= 64 && d.k % 8 == 0 && d.lda % 8 == 0 && d.ldb % 8 == 0 &&

@@ -296,8 +296,6 @@ hipError_t launch_mp(const MopaArgs &g, const EpArgs &ep, int epv, hipStream_t s
     return hipGetLastError();
 }
 
-}  // namespace
-
 // The tile's rows, or 0 where gemm_kernel is faster. Rounds: a workgroup fills a
 // compute unit, so a product takes as many passes over the chip as its tiles
 // make. A pass over 4096 depths, us:
@@ -318,6 +316,13 @@ int mopa_tile(const WDev &w, size_t m) {
                  rk = (mt * ((w.n + 127) / 128) + cus - 1) / cus;
     if (w.kind == W_Q1) return r256 * 5 < r128 * 4 ? 256 : 128;
     return r256 * 5 < rk * 4 ? 256 : 0;
+}
+
+}  // namespace
+
+TileDims gemm_mopa_tile(const WDev &w, size_t m) {
+    const uint32_t rows = (uint32_t)mopa_tile(w, m);
+    return {rows, rows ? (uint32_t)MP : 0u};
 }
 
 bool gemm_mopa_supported(const WDev &w, size_t m, long lhs_cs, long lhs_rs, const uint16_t *lhs) {

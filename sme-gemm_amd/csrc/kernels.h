@@ -75,6 +75,12 @@ hipError_t launch_lowbit_gemv(const WDev &w, size_t m, uint16_t *dst, const uint
 // 64, 128 or 256. lowbit_gemm_bytes is its scratch, 0 where it does not serve.
 constexpr size_t LOWBIT_GEMM_ROWS = 9;
 size_t lowbit_gemm_bytes(const WDev &w, size_t m);
+// The output tile of a product: rows x columns a workgroup, 0 x 0 where its
+// kernel does not serve.
+struct TileDims {
+    uint32_t rows, cols;
+};
+TileDims lowbit_gemm_tile(const WDev &w, size_t m);
 hipError_t launch_lowbit_gemm(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs, const EpArgs &ep,
                               void *scratch, hipStream_t s);
 
@@ -114,11 +120,13 @@ struct DenseGemm {
     bool read_dst;
 };
 bool gemm_dense_supported(const DenseGemm &d);
+TileDims gemm_dense_tile_dims(size_t m, size_t n, size_t k);
 hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hipStream_t s);
 
 // The f16 GEMM over low-bit weights (gemm_mopa.cuh); launch_gemm uses it
 // whenever gemm_mopa_supported holds.
 bool gemm_mopa_supported(const WDev &w, size_t m, long lhs_cs, long lhs_rs, const uint16_t *lhs);
+TileDims gemm_mopa_tile(const WDev &w, size_t m);
 hipError_t launch_gemm_mopa(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
                             long lhs_rs, float beta, const EpArgs &ep, hipStream_t s);
 

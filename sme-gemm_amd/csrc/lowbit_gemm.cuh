@@ -45,7 +45,7 @@ struct LgArgs {
     uint32_t m, n, n_pad;
     uint32_t nsteps, nbk;   // 256-depth steps, blocks that hold depths below k
     uint32_t mt16;          // 16-row tiles of A
-    uint32_t sc_rows, codebook;
+    uint32_t codebook;
     // the compiled store's operands (EpPick's a, b, act, alpha)
     const uint16_t *col_a, *col_b;
     uint32_t act;
@@ -375,13 +375,19 @@ hipError_t launch_lg(const LgArgs &g, const EpArgs &ep, int epv, hipStream_t s) 
 // GEMV launches these calls took before, which read every weight once per 16
 // rows: N = 11008 at 16 / 64 / 512 rows 22.1 / 59.3 / 426.9, here 12.0 / 16.3 /
 // 48.4; N = 4096 at 9 rows 12.0, here 11.5.)
+TileDims lg_tile(size_t mt16, size_t n_pad) {
+    const size_t cols = n_pad / 64, most = (size_t)device_cus() * 11 / 4;
+    for (uint32_t rt : {1u, 2u, 4u})
+        if ((mt16 + rt - 1) / rt * cols <= most) return {16 * rt, 64};
+    return {64, 128};
+}
 template <int KIND, int SPB>
 hipError_t launch_lg_rows(const LgArgs &g, const EpArgs &ep, int epv, hipStream_t s) {
-    const size_t cols = g.n_pad / 64, most = (size_t)device_cus() * 11 / 4;
-    if (g.mt16 * cols <= most) return launch_lg<KIND, SPB, 1, 1, 4>(g, ep, epv, s);
-    if ((g.mt16 + 1) / 2 * cols <= most) return launch_lg<KIND, SPB, 2, 1, 4>(g, ep, epv, s);
-    if ((g.mt16 + 3) / 4 * cols <= most) return launch_lg<KIND, SPB, 4, 1, 3>(g, ep, epv, s);
-    return launch_lg<KIND, SPB, 4, 2, 2>(g, ep, epv, s);
+    const TileDims t = lg_tile(g.mt16, g.n_pad);
+    if (t.cols == 128) return launch_lg<KIND, SPB, 4, 2, 2>(g, ep, epv, s);
+    if (t.rows == 16) return launch_lg<KIND, SPB, 1, 1, 4>(g, ep, epv, s);
+    if (t.rows == 32) return launch_lg<KIND, SPB, 2, 1, 4>(g, ep, epv, s);
+    return launch_lg<KIND, SPB, 4, 1, 3>(g, ep, epv, s);
 }
 
 }  // namespace
@@ -412,6 +418,11 @@ size_t lowbit_gemm_bytes(const WDev &w, size_t m) {
     return lg_q_bytes(w, m) + blocks * ((m + 15) / 16 * 16) * sizeof(float);
 }
 
+TileDims lowbit_gemm_tile(const WDev &w, size_t m) {
+    if (!lowbit_gemm_bytes(w, m)) return {0, 0};
+    return lg_tile((m + 15) / 16, w.n_pad);
+}
+
 hipError_t launch_lowbit_gemm(const WDev &w, size_t m, uint16_t *dst, const uint16_t *lhs, const EpArgs &ep,
                               void *scratch, hipStream_t s) {
     LgArgs g = {};
@@ -426,7 +437,6 @@ hipError_t launch_lowbit_gemm(const WDev &w, size_t m, uint16_t *dst, const uint
     g.nsteps = lg_steps(w);
     g.nbk = (uint32_t)((w.k + w.block - 1) / w.block);
     g.mt16 = (uint32_t)((m + 15) / 16);
-    g.sc_rows = (uint32_t)w.sc_rows;
     g.codebook = w.codebook;
     const EpPick pk = pick_ep(ep);
     g.col_a = pk.a;

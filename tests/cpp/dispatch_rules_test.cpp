@@ -1,6 +1,7 @@
 // The dispatch rules' bounds on sizes whose arrays need not exist: only host
 // code of the launch interface runs, nothing reaches a GPU.
 #include <cstdio>
+#include <cstring>
 
 #include "kernels.h"
 
@@ -32,7 +33,33 @@ static WDev lowbit(int kind, size_t n, size_t k, size_t block) {
 // adds it to its step's base.
 static size_t last_code(const WDev &w) { return cell_col_part(w.n_pad - 1, 0, w.n_pad) * 64 + 3 * 16 + 16; }
 
-int main() {
+// `tiles`: a call a line on stdin ("dense m n k", "lowbit bits block m n k", "mopa
+// bits m n k"), its tile ("rows cols") a line on stdout.
+static int tiles() {
+    char op[16];
+    size_t m, n, k, block;
+    int bits;
+    while (std::scanf("%15s", op) == 1) {
+        TileDims t = {0, 0};
+        if (!std::strcmp(op, "dense")) {
+            if (std::scanf("%zu %zu %zu", &m, &n, &k) != 3) return 1;
+            t = gemm_dense_tile_dims(m, n, k);
+        } else if (!std::strcmp(op, "lowbit")) {
+            if (std::scanf("%d %zu %zu %zu %zu", &bits, &block, &m, &n, &k) != 5) return 1;
+            t = lowbit_gemm_tile(lowbit(bits == 1 ? W_Q1 : W_Q2, n, k, block), m);
+        } else if (!std::strcmp(op, "mopa")) {
+            if (std::scanf("%d %zu %zu %zu", &bits, &m, &n, &k) != 4) return 1;
+            t = gemm_mopa_tile(lowbit(bits == 1 ? W_Q1 : W_Q2, n, k, 128), m);
+        } else {
+            return 1;
+        }
+        std::printf("%u %u\n", t.rows, t.cols);
+    }
+    return 0;
+}
+
+int main(int argc, char **argv) {
+    if (argc > 1 && !std::strcmp(argv[1], "tiles")) return tiles();
     const int kinds[2] = {W_Q2, W_Q1};
     // The many-row GEMM serves a call only where a column's code offset fits the
     // DMA's 32-bit lane offset.

@@ -16,7 +16,9 @@ SHAPES = [(9, 128, 256), (16, 5, 64), (17, 130, 300), (31, 257, 512), (32, 384, 
           (63, 128, 4096), (64, 129, 520), (65, 640, 2049), (130, 300, 1288),
           # 32-row, 64-row and 64 x 128 tiles (more 16-row tiles than the
           # device takes at once), ragged rows and columns
-          (130, 8200, 300), (300, 9001, 256), (400, 16300, 328)]
+          (130, 8200, 300), (300, 8900, 256), (300, 9001, 256), (400, 16300, 328)]
+# the same three tiles, one block deep (test_host_logic.py holds the rule to both)
+WIDE = [(130, 8200, 128), (300, 8900, 128), (400, 16300, 128)]
 BOOKS = [(-1, 0, 1, 0), (-2, -1, 1, 2), (-128, 127, 3, -7)]
 
 
@@ -73,6 +75,26 @@ def test_many_rows_epilogue_bits(smg, orc, graph):
                         [(3, 0, 0.0, r, 0), (6, 0, 0.0, t, n)], 5),
     }[graph]
     _both(smg, orc, a, codes2, signs, scales, m, n, k, block, (-1, 0, 1, 0), ep, nodes, act)
+
+
+@pytest.mark.parametrize("graph", ["scale_bias_gelu", "interpreted"])
+@pytest.mark.parametrize("m,n,k", WIDE)
+def test_wide_tiles_epilogue_bits(smg, orc, m, n, k, graph):
+    """The compiled and the interpreted store of the tiles past 16 rows."""
+    block = 128
+    rng = np.random.default_rng(m)
+    a, codes, scales = _inputs(orc, rng, m, n, k, block, 2)
+    b = orc.f32_to_f16(rng.uniform(-4, 4, n).astype(np.float32))
+    s = orc.f32_to_f16(rng.uniform(0.5, 1.5, n).astype(np.float32))
+    r = orc.f32_to_f16(rng.uniform(0.5, 1.5, m).astype(np.float32))
+    if graph == "interpreted":
+        ep, nodes, act = smg.Epilogue().mul_row(r).add_col(b).relu(), [(3, 0, 0.0, r, 0), (4, 0, 0.0, b, 0)], 1
+    else:
+        ep, nodes, act = smg.Epilogue().mul_col(s).add_col(b).gelu(), [(5, 0, 0.0, s, 0), (4, 0, 0.0, b, 0)], 2
+    w = smg.Q2Weights(codes, scales, n, k, smg.Q2Params(block))
+    got = np.full(m * n, 0x4880, np.uint16)
+    smg.matmul_q2_ep(a, w, got, m, ep)
+    assert np.array_equal(got, orc.matmul_lowbit_ep(2, a, codes, scales, m, n, k, block, nodes, act))
 
 
 def test_many_rows_special_activations(smg, orc):

@@ -38,9 +38,12 @@ def _weights(smg, bits, n, k, block, seed):
 
 # rows x columns that reach 128-row tiles (1-bit) and 256-row ones (both kinds:
 # more than one pass of the chip's units with the smaller tiles)
-@pytest.mark.parametrize("bits,m,n,k,block", [
+SHAPES = [
     (1, 129, 1, 64, 64), (1, 200, 300, 200, 128), (1, 257, 129, 520, 64), (1, 385, 1000, 584, 256),
-    (1, 2049, 4097, 136, 128), (2, 2049, 4097, 136, 128), (2, 2300, 4000, 328, 64), (2, 4096, 4096, 64, 256)])
+    (1, 2049, 4097, 136, 128), (2, 2049, 4097, 136, 128), (2, 2300, 4000, 328, 64), (2, 4096, 4096, 64, 256)]
+
+
+@pytest.mark.parametrize("bits,m,n,k,block", SHAPES)
 @pytest.mark.parametrize("ep", [False, True])
 def test_mopa_gemm(smg, bits, m, n, k, block, ep):
     import torch

@@ -104,16 +104,48 @@ def _library_objects():
     return objs
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
-def test_dispatch_rules(tmp_path):
-    """The launch interface's rules (csrc/kernels.h) at the edges of their ranges,
-    on the host alone."""
-    drv, exe = str(tmp_path / "drv.o"), str(tmp_path / "dispatch_rules_test")
+@pytest.fixture(scope="module")
+def dispatch_rules(tmp_path_factory):
+    """tests/cpp/dispatch_rules_test.cpp linked with the library's objects."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("needs hipcc")
+    tmp = tmp_path_factory.mktemp("dispatch")
+    drv, exe = str(tmp / "drv.o"), str(tmp / "dispatch_rules_test")
     subprocess.run([HIPCC, "--offload-arch=gfx950", "-O1", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                     "-packed-fp32-ops", "-I", os.path.join(ROOT, "sme-gemm_amd", "csrc"), "-x", "hip", "-c",
                     os.path.join(CPP, "dispatch_rules_test.cpp"), "-o", drv], check=True, timeout=300,
                    capture_output=True)
     subprocess.run([HIPCC, "--offload-arch=gfx950", *_library_objects(), drv, "-o", exe, "-lpthread"], check=True,
                    timeout=300, capture_output=True)
-    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    return exe
+
+
+def test_dispatch_rules(dispatch_rules):
+    """The launch interface's rules (csrc/kernels.h) at the edges of their ranges,
+    on the host alone."""
+    r = subprocess.run([dispatch_rules], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "dispatch rules ok" in r.stdout, r.stdout + r.stderr
+
+
+def _tiles(exe, calls):
+    """Each call's tile, at the 256 compute units the rules count without a GPU."""
+    text = "".join(" ".join(map(str, c)) + "\n" for c in calls)
+    r = subprocess.run([exe, "tiles"], input=text, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    return [tuple(map(int, x.split())) for x in r.stdout.splitlines()]
+
+
+def test_gpu_shapes_reach_every_tile(dispatch_rules):
+    """The GPU tests' shapes take the tiles they are there for."""
+    import test_gpu_dense as dense
+    import test_gpu_lowbit_gemm as low
+    import test_gpu_mopa as mopa
+    assert _tiles(dispatch_rules, [("dense", *s) for s in dense.TILES]) == [
+        (256, 256), (128, 256), (64, 128), (64, 64), (64, 64), (32, 64)]
+    for bits in (1, 2):
+        for block in (64, 128, 256):
+            got = set(_tiles(dispatch_rules, [("lowbit", bits, block, *s) for s in low.SHAPES]))
+            assert got >= {(16, 64), (32, 64), (64, 64), (64, 128)}, (bits, block, got)
+        assert _tiles(dispatch_rules, [("lowbit", bits, 128, *s) for s in low.WIDE]) == [(32, 64), (64, 64), (64, 128)]
+    got = _tiles(dispatch_rules, [("mopa", *s[:4]) for s in mopa.SHAPES])
+    assert got == [(128, 256)] * 4 + [(256, 256)] * 4, got
