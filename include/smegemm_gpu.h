@@ -52,7 +52,8 @@ extern "C" {
  * callers rely on to take their portable path on a non-zero return
  * (src/kernels/q4/matmul.rs:85-89). Buffers a call allocated earlier
  * (the host-call staging area, the device-form scratch pool) are kept and
- * reused, so only a first allocation or a growth fails. */
+ * reused, so only a first allocation or a growth fails. A value N above 1 fails
+ * the allocations of more than N bytes alone. */
 
 /* ---- epilogue ABI: byte-identical to csrc/epilogue.h:136-236 -------------- */
 enum ep_act {

@@ -86,15 +86,22 @@ thread_local Ctx g_ctx;
 // hipMalloc, or a forced failure while the environment has
 // SMG_TEST_FAIL_ALLOC=1: a test hook for the reference's contract that a call
 // whose allocation fails returns non-zero and leaves its output untouched, so
-// the caller takes its portable path (src/kernels/q4/matmul.rs:85-89). The
+// the caller takes its portable path (src/kernels/q4/matmul.rs:85-89). A larger
+// value N fails the allocations past N bytes alone, as a full device does. The
 // variable is read at every allocation.
 hipError_t dev_malloc(void **p, size_t bytes) {
     const char *f = std::getenv("SMG_TEST_FAIL_ALLOC");
-    if (f && f[0] == '1') {
+    const unsigned long long most = f ? std::strtoull(f, nullptr, 10) : 0;
+    if (most == 1) {
         *p = nullptr;
         return hipErrorOutOfMemory;
     }
-    return hipMalloc(p, bytes);
+    if (most > 1 && bytes > most) bytes = (size_t)1 << 50;  // more than any device has
+    const hipError_t e = hipMalloc(p, bytes);
+    // the caller reports it or does without: left in place, the next launch's
+    // check would take it for its own
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 int ctx_for(int device, size_t bytes, Ctx **out) {
@@ -170,9 +177,7 @@ struct PackAlloc {
     };
     void *acquire(int device, size_t bytes) {
         Relaxed r;
-        void *p = HipDevAlloc().acquire(device, bytes);
-        if (!p) (void)hipGetLastError();
-        return p;
+        return HipDevAlloc().acquire(device, bytes);
     }
     void release(int, void *p) {
         Relaxed r;
@@ -1448,16 +1453,25 @@ static int lowbit_host(int kind, bool mopa, size_t m, const smg_weights *w, uint
     const size_t n = w->d.n, k = w->d.k;
     if (m == 0 || n == 0) return SMG_OK;  // lowbit/matmul.rs:318-324
     const WDev d = w->d;
-    const size_t scratch = mopa ? 0 : lowbit_scratch_bytes(d, m);
+    size_t scratch = mopa ? 0 : lowbit_scratch_bytes(d, m);
     const char *name = mopa ? (kind == W_Q2 ? "gemm_gpu_f16f16_q2" : "gemm_gpu_f16f16_q1")
                             : (kind == W_Q2 ? "gemm_gpu_f16_q2" : "gemm_gpu_f16_q1");
-    return host_call(name, w->device, m, n, k, dst, m * n, false, lhs, m * k, ep, scratch,
-                     [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
-                         const hipError_t e = mopa ? launch_gemm(d, m, dd, 1, (long)n, dl, 1, (long)k, 1.0f, p.fused,
-                                                                 false, s)
-                                                   : launch_lowbit_gemv(d, m, dd, dl, p.fused, sc, scratch, s);
-                         return e == hipSuccess ? plan_tail(p, dd, 1, (long)n, m, n, false, s) : e;
-                     });
+    auto call = [&]() {
+        return host_call(name, w->device, m, n, k, dst, m * n, false, lhs, m * k, ep, scratch,
+                         [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
+                             const hipError_t e = mopa ? launch_gemm(d, m, dd, 1, (long)n, dl, 1, (long)k, 1.0f, p.fused,
+                                                                     false, s)
+                                                       : launch_lowbit_gemv(d, m, dd, dl, p.fused, sc, scratch, s);
+                             return e == hipSuccess ? plan_tail(p, dd, 1, (long)n, m, n, false, s) : e;
+                         });
+    };
+    rc = call();
+    if (rc != SMG_ENOMEM || !scratch) return rc;
+    // no room for the GEMM's rows: the GEMV's may fit
+    const size_t less = lowbit_scratch_bytes(d, m, nullptr, scratch - 1);
+    if (less >= scratch) return rc;
+    scratch = less;
+    return call();
 }
 
 int gemm_gpu_f16_q2(size_t m, const smg_weights *w, uint16_t *dst, const uint16_t *lhs,
@@ -1497,28 +1511,34 @@ static int packed_host(bool bf16, size_t m, size_t n, size_t k, uint16_t *dst, l
     // add_dst step)
     const bool tail_add = read_dst && ep && ep->n_nodes > (uint32_t)EP_FUSED;
     // (the staged copy of A is 256-byte aligned)
-    const size_t ab = tail_add ? 0 : dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs);
-    return host_call(bf16 ? "gemm_gpu_b16b16_run_packed" : "gemm_gpu_f16f16_run_packed", b->device,
-                     m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, lhs_elems, ep, tail_add ? m * n * 2 : ab,
-                     [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
-                         if (ab) {
-                             const hipError_t e = launch_gemm_pack_a(d, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta,
-                                                                     p.fused, bf16, (uint16_t *)sc, s, read_dst != 0,
-                                                                     alpha);
+    size_t ab = tail_add ? 0 : dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs);
+    auto call = [&]() {
+        return host_call(bf16 ? "gemm_gpu_b16b16_run_packed" : "gemm_gpu_f16f16_run_packed", b->device,
+                         m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, lhs_elems, ep, tail_add ? m * n * 2 : ab,
+                         [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
+                             if (ab) {
+                                 const hipError_t e = launch_gemm_pack_a(d, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta,
+                                                                         p.fused, bf16, (uint16_t *)sc, s, read_dst != 0,
+                                                                         alpha);
+                                 return e == hipSuccess ? plan_tail(p, dd, dst_cs, dst_rs, m, n, bf16, s) : e;
+                             }
+                             if (tail_add) {
+                                 uint16_t *prod = (uint16_t *)sc;
+                                 const hipError_t e = launch_gemm(d, m, prod, 1, (long)n, dl, lhs_cs, lhs_rs, beta,
+                                                                  p.fused, bf16, s, false, 0.0f);
+                                 return e == hipSuccess ? launch_ep_tail(prod, (long)n, 1, dd, dst_rs, dst_cs, m, n, alpha,
+                                                                         true, p.tail, bf16, s)
+                                                        : e;
+                             }
+                             const hipError_t e = launch_gemm(d, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, p.fused,
+                                                              bf16, s, read_dst != 0, alpha);
                              return e == hipSuccess ? plan_tail(p, dd, dst_cs, dst_rs, m, n, bf16, s) : e;
-                         }
-                         if (tail_add) {
-                             uint16_t *prod = (uint16_t *)sc;
-                             const hipError_t e = launch_gemm(d, m, prod, 1, (long)n, dl, lhs_cs, lhs_rs, beta,
-                                                              p.fused, bf16, s, false, 0.0f);
-                             return e == hipSuccess ? launch_ep_tail(prod, (long)n, 1, dd, dst_rs, dst_cs, m, n, alpha,
-                                                                     true, p.tail, bf16, s)
-                                                    : e;
-                         }
-                         const hipError_t e = launch_gemm(d, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, p.fused,
-                                                          bf16, s, read_dst != 0, alpha);
-                         return e == hipSuccess ? plan_tail(p, dd, dst_cs, dst_rs, m, n, bf16, s) : e;
-                     });
+                         });
+    };
+    rc = call();
+    if (rc != SMG_ENOMEM || !ab) return rc;
+    ab = 0;  // no room for A's copy: the product reads A as it is
+    return call();
 }
 
 int gemm_gpu_f16f16_run_packed(size_t m, size_t n, size_t k, uint16_t *dst, long dst_cs,
@@ -1594,32 +1614,39 @@ static int run_host(bool bf16, const char *name, size_t m, size_t n, size_t k, u
     const bool dense_out = (dst_cs == 1 && (size_t)dst_rs == n) || (dst_rs == 1 && (size_t)dst_cs == m);
     const float alpha = half_bits_to_float(alpha_bits, bf16), beta = half_bits_to_float(beta_bits, bf16);
     // scratch: the packed B, then the packed A where it is needed, then B as given
-    const size_t ab = dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs), raw_at = dense_bytes + round_up(ab, 256);
-    return host_call(name, device, m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, footprint(m, lhs_rs, k, lhs_cs),
-                     nullptr, raw_at + rhs_elems * 2,
-                     [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
-                         const EpArgs &ea = p.fused;  // no op-graph on these entry points
-                         uint16_t *dense = (uint16_t *)sc, *raw = (uint16_t *)((uint8_t *)sc + raw_at);
-                         if (rhs_elems) {
-                             const hipError_t e = hipMemcpyAsync(raw, rhs, rhs_elems * 2, hipMemcpyHostToDevice, s);
+    size_t ab = dense_pack_a_bytes(d, m, nullptr, lhs_cs, lhs_rs);
+    auto call = [&]() {
+        const size_t raw_at = dense_bytes + round_up(ab, 256);
+        return host_call(name, device, m, n, k, dst, dst_elems, !dense_out || read_dst, lhs, footprint(m, lhs_rs, k, lhs_cs),
+                         nullptr, raw_at + rhs_elems * 2,
+                         [&](uint16_t *dd, const uint16_t *dl, const EpPlan &p, void *sc, hipStream_t s) {
+                             const EpArgs &ea = p.fused;  // no op-graph on these entry points
+                             uint16_t *dense = (uint16_t *)sc, *raw = (uint16_t *)((uint8_t *)sc + raw_at);
+                             if (rhs_elems) {
+                                 const hipError_t e = hipMemcpyAsync(raw, rhs, rhs_elems * 2, hipMemcpyHostToDevice, s);
+                                 if (e != hipSuccess) return e;
+                             }
+                             DenseGemm dg;
+                             if (strided_direct(&dg, m, n, k, dd, dst_cs, dst_rs, read_dst, dl, lhs_cs, lhs_rs, raw, rhs_cs,
+                                                rhs_rs, alpha, beta))
+                                 return launch_gemm_dense(dg, ea, bf16, s);
+                             hipError_t e = launch_pack_dense_strided(raw, rhs_rs, rhs_cs, n, k, d.n_pad, d.k_pad,
+                                                                      dense, s);
                              if (e != hipSuccess) return e;
-                         }
-                         DenseGemm dg;
-                         if (strided_direct(&dg, m, n, k, dd, dst_cs, dst_rs, read_dst, dl, lhs_cs, lhs_rs, raw, rhs_cs,
-                                            rhs_rs, alpha, beta))
-                             return launch_gemm_dense(dg, ea, bf16, s);
-                         hipError_t e = launch_pack_dense_strided(raw, rhs_rs, rhs_cs, n, k, d.n_pad, d.k_pad,
-                                                                  dense, s);
-                         if (e != hipSuccess) return e;
-                         WDev w = d;
-                         w.dense = dense;
-                         if (ab)
-                             return launch_gemm_pack_a(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16,
-                                                       (uint16_t *)((uint8_t *)sc + dense_bytes), s, read_dst != 0,
-                                                       alpha);
-                         return launch_gemm(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16, s,
-                                            read_dst != 0, alpha);
-                     });
+                             WDev w = d;
+                             w.dense = dense;
+                             if (ab)
+                                 return launch_gemm_pack_a(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16,
+                                                           (uint16_t *)((uint8_t *)sc + dense_bytes), s, read_dst != 0,
+                                                           alpha);
+                             return launch_gemm(w, m, dd, dst_cs, dst_rs, dl, lhs_cs, lhs_rs, beta, ea, bf16, s,
+                                                read_dst != 0, alpha);
+                         });
+    };
+    const int rc = call();
+    if (rc != SMG_ENOMEM || !ab) return rc;
+    ab = 0;  // no room for A's copy: the product reads A as it is
+    return call();
 }
 
 int gemm_gpu_f16f16_run(size_t m, size_t n, size_t k, uint16_t *dst, long dst_cs, long dst_rs, int read_dst,
@@ -1771,12 +1798,19 @@ int smg_lowbit_matmul_dev(size_t m, const smg_weights *w, uint16_t *dst, const u
     if (rc) return rc;
     if ((rc = check_dev_ptrs("smg_lowbit_matmul_dev", w->device, stream, ep_p, {dst, lhs}))) return rc;
     const EpArgs &ea = ep_p.fused;
-    const size_t sb = lowbit_scratch_bytes(w->d, m, &ea);
+    size_t sb = lowbit_scratch_bytes(w->d, m, &ea);
     void *scratch = nullptr;
     if (sb) {
         // several rows (or blocks past one in-kernel pass): the activations
-        // are quantized once into a buffer of this stream's own
-        scratch = dev_pool().get(w->device, stream, sb);
+        // are quantized once into a buffer of this stream's own; where the
+        // GEMM's whole tiles of rows would have to grow it while the stream is
+        // captured, or do not fit the device, the GEMV's rows if they do
+        const size_t less = lowbit_scratch_bytes(w->d, m, &ea, sb - 1);
+        scratch = dev_pool().find(w->device, stream, sb);
+        if (!scratch && less < sb && stream_capturing(stream) && (scratch = dev_pool().find(w->device, stream, less)))
+            sb = less;
+        if (!scratch) scratch = dev_pool().get(w->device, stream, sb);
+        if (!scratch && less < sb && (scratch = dev_pool().get(w->device, stream, less))) sb = less;
         if (!scratch) return fail(SMG_ENOMEM, "smg_lowbit_matmul_dev: scratch hipMalloc");
     }
     hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, scratch, sb, (hipStream_t)stream);
