@@ -445,36 +445,17 @@ class Epilogue:
                     raise ValueError("tensor must hold m*n elements (stride ld)")
 
     def desc(self, n: int):
-        """resolve_nodes (src/exec/scalar.rs:28-53): tensor ld 0 -> n, the
-        trailing activation appended as a final ACT node. Returns
-        (EpDesc16 or None, keepalive)."""
-        nodes = []
-        keep = []
-        for op, aux, scalar, v, ld in self.nodes:
-            ptr = None
-            if v is not None:
-                if not _is_dev(v):
-                    v = _host_operand(v, self.bf16)
-                keep.append(v)
-                ptr = _ptr(v)
-            if op in _TENSOR and ld == 0:
-                ld = n
-            nodes.append(EpNode(op, aux, scalar, ptr, ld))
-        if self.act is not None:
-            nodes.append(EpNode(8, self.act, 0.0, None, 0))
-        if not nodes:
-            return None, keep
-        arr = (EpNode * len(nodes))(*nodes)
-        keep.append(arr)
-        d = EpDesc16(len(nodes), C.cast(arr, C.POINTER(EpNode)))
-        keep.append(d)
-        return d, keep
+        """packed() as ctypes structures: (EpDesc16 or None, keepalive)."""
+        addr, keep = self.packed(n)
+        return (None if addr is None else EpDesc16.from_address(addr)), keep
 
     def packed(self, n: int):
-        """desc(n) for a call: the descriptor's address (None for an empty graph)
-        and what keeps it alive -- one buffer of the descriptor and its nodes
-        (built as ctypes structures they took 2.1 us for bias + activation,
-        packed 1.0), and the operands."""
+        """resolve_nodes (src/exec/scalar.rs:28-53) for a call: tensor ld 0 -> n,
+        the trailing activation appended as a final ACT node. Returns the
+        descriptor's address (None for an empty graph) and what keeps it alive
+        -- one buffer of the descriptor and its nodes (built as ctypes
+        structures they took 2.1 us for bias + activation, packed 1.0), and the
+        operands."""
         count = len(self.nodes) + (self.act is not None)
         if not count:
             return None, []

@@ -369,15 +369,23 @@ def test_host_slice_arrays_in_the_mirror():
 
 
 def test_packed_descriptor_is_desc():
-    """The packed form a call passes holds desc()'s bytes (the node pointer
-    aside), for every operand class, a stride and a trailing activation."""
+    """The buffer a call passes holds the nodes as EpDesc16 and EpNode lay them
+    out, for every operand class, a stride, scalars past f32's range (infinite
+    after T's rounding) and a trailing activation."""
     import smegemm as smg
     t, r, c = (np.arange(x, dtype=np.uint16) for x in (60, 6, 10))
-    ep = smg.Epilogue().mul_scalar(0.5).add_row(r).mul_col(c).add_tensor(t).max_tensor(t, ld=10).elu(0.3).silu()
-    d, keep = ep.desc(10)
-    addr, keep2 = ep.packed(10)
+    with np.errstate(over="ignore"):
+        ep = (smg.Epilogue().mul_scalar(0.5).add_row(r).mul_col(c).add_tensor(t).max_tensor(t, ld=12).elu(0.3)
+              .add_scalar(1e39).leaky_relu(-1e39).silu())
+    inf = float("inf")
+    want = [(1, 0, 0.5, None, 0), (2, 0, 0.0, r, 0), (5, 0, 0.0, c, 0), (6, 0, 0.0, t, 10), (21, 0, 0.0, t, 12),
+            (8, 20, float(np.float32(0.3)), None, 0), (0, 0, inf, None, 0), (8, 6, -inf, None, 0), (8, 3, 0.0, None, 0)]
+    addr, keep = ep.packed(10)
     got = C.cast(addr, C.POINTER(smg.EpDesc16)).contents
-    assert got.n_nodes == d.n_nodes == 7
-    size = C.sizeof(smg.EpNode) * 7
-    assert C.string_at(got.nodes, size) == C.string_at(d.nodes, size)
+    assert got.n_nodes == len(want)
+    for i, (op, aux, scalar, v, ld) in enumerate(want):
+        nd = got.nodes[i]
+        assert (nd.op, nd.aux, nd.scalar, nd.ptr, nd.ld) == (op, aux, scalar, None if v is None else v.ctypes.data, ld)
+    d, keep2 = ep.desc(10)
+    assert d.n_nodes == len(want) and d.nodes[4].ld == 12
     assert smg.Epilogue().packed(10) == (None, [])
