@@ -923,9 +923,10 @@ __global__ void __launch_bounds__(AP_T) attn_rows_mfma(AttnArgs a) {
 // LDS. Masks (scores, and values past the unit's last position, so that no
 // row's probability of zero meets them) only where a wave's keys reach the
 // unit's own positions.
-// What bounds it: the vector instructions (16 of them 2^x, and the rescale's 64
-// in most early blocks) and 32 products a wave and block, two waves a SIMD, one
-// barrier a block. Measured (us, one MI355X, q's rounding pass included;
+// What bounds it: the vector instructions (seven a product: 16 of a wave's and
+// block's are 2^x, and 64 the rescale in most early blocks), 46 % of the kernel's
+// issue cycles, beside products of 21 %, two waves a SIMD, one barrier a block.
+// Measured (us, one MI355X, q's rounding pass included;
 // attn_rows_mfma, one wave a SIMD with 160 KB of LDS traffic a 64-key block,
 // before): 512 rows after 4096 positions, 32 heads of 128 over 8 KV heads 128 ->
 // 67, over 32 KV heads 353 -> 71; 1024 rows after 8192 367 -> 221; 2048 rows, 16

@@ -3,8 +3,10 @@
 // B [n][ldb] (column j's K at row j): Packed<f16> / Packed<bf16>
 // (Gemm::new(&a, &packed, m)...run(), replacing run_packed,
 // csrc/gemm_half.h:1054) and the strided gemm_f16 / gemm_bf16
-// (src/kernels/f16.rs:126-204, bf16.rs:140-200). K in multiples of 8 with
-// 16-byte-aligned rows; every other case goes to gemm_kernel (gemm_mfma.hip).
+// (src/kernels/f16.rs:126-204, bf16.rs:140-200). K from 64 in multiples of 8 with
+// 16-byte-aligned rows; an A of any other kind is packed into such rows first
+// where that pays and there is scratch for it (dense_pack_a_bytes), else the call
+// goes to gemm_kernel (gemm_mfma.hip).
 // Products are v_mfma_f32_16x16x32_{f16,bf16} accumulating in f32, the portable
 // path's accumulator type (src/reference.rs:349-387).
 //
@@ -26,9 +28,11 @@
 // where 256-row tiles leave compute units idle.)
 // gemm_dense_tile: smaller tiles of four waves for smaller products.
 // What bounds them: 8192^3 runs at 1.42 PF/s, 1.5 us a step of 64 depths where
-// the products alone are 0.85 us at the nominal clock; the fragment reads and
-// the refill take the LDS about as long as the products take the matrix cores,
-// and the slots' barriers keep the two from overlapping fully.
+// the products alone are 0.85 us at the nominal clock. Counters at 4096^3: the
+// matrix cores busy 60 % of the kernel's cycles, waves waiting for an issue slot
+// 42 % of theirs and for data or a barrier 28 %. The smaller tiles wait: 64 x 128 at
+// 1000 x 3000 x 2000, the matrix cores busy 15 %, waves waiting for the next stage
+// 56 %.
 #include <algorithm>
 #include <type_traits>
 

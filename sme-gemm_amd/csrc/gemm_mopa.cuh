@@ -18,7 +18,8 @@
 // quarter of A's stage is refilled as in gemm_dense_big, a step's codes six
 // phases ahead.
 // What bounds it: the slots that expand, which take longer than the products
-// beside them (128 rows: eight 16x16x32 products a slot). 4096 depths,
+// beside them (128 rows: eight 16x16x32 products a slot; 3.5 vector instructions a
+// product, the matrix cores busy 29 % of the kernel's cycles). 4096 depths,
 // gemm_kernel -> this (us): 1-bit 512 x 14336 82 -> 70 (with bias and silu 87 ->
 // 74), 1024 x 14336 160 -> 97, 4096 x 4096 178 -> 105; 2-bit 1024 x 14336 147 ->
 // 104, 4096 x 4096 160 -> 116.

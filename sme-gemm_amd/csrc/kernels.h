@@ -14,8 +14,8 @@ enum WKind { W_Q4 = 4, W_Q2 = 2, W_Q1 = 1, W_F16 = 16, W_BF16 = 17 };
 struct WDev {
     int kind;
     size_t n, k, block;
-    size_t n_pad;     // columns padded to a multiple of 64
-    size_t nchunks;   // chunks along K (Q4: 32 depths, Q2: 64, Q1: 128)
+    size_t n_pad;     // columns padded to a multiple of 128
+    size_t nchunks;   // chunks along K (Q4: 32 depths, Q2: 256, Q1: 512)
     size_t sc_rows;   // rows of the scale array
     const uint8_t *codes;   // Q4 nibbles / Q2 codes / Q1 signs
     const uint16_t *scales;

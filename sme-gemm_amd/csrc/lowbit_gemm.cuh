@@ -21,7 +21,8 @@
 //   products.
 // What bounds it: the fold's three vector instructions an output and block
 //   (convert, scale product, fma) and the expansion, about twice the matrix
-//   cores' time for the same block; so the expansion is shared by RT row
+//   cores' time for the same block (2-bit 512 x 11008 x 4096: vector issue 57 % of
+//   the kernel's cycles, products 19 %); so the expansion is shared by RT row
 //   tiles and several waves a SIMD overlap one's fold with another's
 //   products.
 #include <algorithm>
@@ -366,15 +367,17 @@ hipError_t launch_lg(const LgArgs &g, const EpArgs &ep, int epv, hipStream_t s) 
 // The tile: the smallest whose workgroups are at most 11/4 of the compute
 // units. Few rows or columns run many small tiles with deep rings (a step's
 // latency is what they wait for); past that a larger tile's shared expansion
-// and fragment reads win. Measured on 256 compute units, K = 4096 (us, tiles
-// of 16x64 / 32x64 / 64x64 / 64x128 rows x columns): 2-bit N = 11008 at 64
+// and fragment reads win. Measured on 256 compute units, K = 4096, blocks of 128
+// (us, tiles of 16x64 / 32x64 / 64x64 / 64x128 rows x columns): 2-bit N = 11008 at 64
 // rows 16.3 / 16.4 / 18.0 / 24.0, at 128 rows 25.2 / 20.9 / 22.6 / 25.3, at 256
 // rows 39.0 / 34.9 / 34.3 / 36.6, at 512 rows 69.8 / 57.0 / 56.2 / 48.4; N =
 // 4096 at 64 rows 12.2 / 14.3 / 17.5 / 23.7, at 512 rows 32.7 / 29.6 / 25.5 /
 // 27.8; 1-bit N = 14336 at 512 rows 148.9 / 88.2 / 67.6 / 62.6. (The 16-row
 // GEMV launches these calls took before, which read every weight once per 16
-// rows: N = 11008 at 16 / 64 / 512 rows 22.1 / 59.3 / 426.9, here 12.0 / 16.3 /
-// 48.4; N = 4096 at 9 rows 12.0, here 11.5.)
+// rows: N = 11008 at 16 / 64 / 512 rows 22.1 / 59.3 / 424, here 12.0 / 16.3 /
+// 46.4; N = 4096 at 9 rows 11.7, here 11.7. Blocks of 64 and 256, the same rule,
+// GEMV and here: N = 5000, K = 4096 at 9 / 64 / 130 rows 18.8 / 42.4 / 84.2 and 12.5 /
+// 14.0 / 19.4, 14.1 / 28.8 / 56.3 and 12.2 / 13.5 / 16.2.)
 TileDims lg_tile(size_t mt16, size_t n_pad) {
     const size_t cols = n_pad / 64, most = (size_t)device_cus() * 11 / 4;
     for (uint32_t rt : {1u, 2u, 4u})
@@ -392,9 +395,10 @@ hipError_t launch_lg_rows(const LgArgs &g, const EpArgs &ep, int epv, hipStream_
 
 }  // namespace
 
-// Calls the 16-row GEMV takes no longer than the GEMM: blocks of 256 (a GEMV
-// wave's own products of a block, and a fold a 256-depth step here) past 2048
-// depths, few rows, and GEMV workgroups (16 rows x 16 columns) that fit the
+// Calls the 16-row GEMV takes no longer than the GEMM: blocks of 256 (9 rows x 700
+// x 8000 take the GEMV 21.8, 18.7 and 16.0 us with blocks of 64, 128 and 256, its
+// folds being its longest step, the GEMM 20.4, 18.4 and 18.8) past 2048 depths, few
+// rows, and GEMV workgroups (16 rows x 16 columns) that fit the
 // compute units once, so that no weight is waited for twice. 2-bit, us, GEMV and
 // GEMM: 9 rows x 700 x 8000 16.0 / 18.8, 32 x 2048 x 4096 12.2 / 12.5, 48 x 700 x
 // 4096 12.3 / 13.0; the other side: 33 x 2048 x 8000 20.8 / 18.6 (a second round),
