@@ -57,7 +57,11 @@ struct LgArgs {
 // (src/kernels/lowbit/matmul.rs:354-371). Rows past m and depths past k are
 // zero. The packed-u16 maximum of |a|'s bits orders as the values do, with NaN
 // above infinity, so a NaN anywhere makes amax NaN as the reference's does.
-template <int SPB>
+// VEC: rows of whole, 16-byte-aligned groups of 8. Other rows are read 64
+// consecutive depths a wave's load and turned through LDS: a lane's own 16 depths
+// read element by element touched 64 places a load, and took a call of few rows
+// and columns up to 3 us longer (2-bit 64 x 700 x 2001, blocks of 256).
+template <int SPB, bool VEC>
 __global__ void __launch_bounds__(256) lowbit_quant_frag(const uint16_t *lhs, uint32_t m, uint32_t k, uint32_t nslab,
                                                          uint32_t mt16, uint32_t nbk, int8_t *q, float *s) {
     const uint32_t w = blockIdx.x * 4 + threadIdx.x / 64;
@@ -66,13 +70,37 @@ __global__ void __launch_bounds__(256) lowbit_quant_frag(const uint16_t *lhs, ui
     const int lane = threadIdx.x % 64, gq = lane / 16, c = lane % 16;
     const uint32_t row = mt * 16 + c;
     const rsrc_t ar = make_rsrc(lhs, m * k * 2u);
-    const bool vec = (k & 7) == 0 && ((uintptr_t)lhs & 15) == 0;
     uint4 a[SPB][2];
+    if constexpr (VEC) {
 #pragma unroll
-    for (int u = 0; u < SPB; u++) {
-        const uint32_t d = (blk * SPB + u) * LB_SLAB + 16 * gq;
-        a[u][0] = load_row8(ar, row, m, k, d, vec);
-        a[u][1] = load_row8(ar, row, m, k, d + 8, vec);
+        for (int u = 0; u < SPB; u++) {
+            const uint32_t d = (blk * SPB + u) * LB_SLAB + 16 * gq;
+            a[u][0] = load_row8(ar, row, m, k, d, true);
+            a[u][1] = load_row8(ar, row, m, k, d + 8, true);
+        }
+    } else {
+        constexpr int RS = SPB * LB_SLAB + 8;  // halfs a staged row
+        __shared__ __align__(16) uint16_t rows[4][16 * RS];
+        uint16_t *st = rows[threadIdx.x / 64];  // the wave's own
+        uint16_t e[16][SPB];
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+            for (int u = 0; u < SPB; u++) {
+                const uint32_t rr = mt * 16 + r, d = (blk * SPB + u) * LB_SLAB + lane;
+                e[r][u] = bload2(ar, rr < m && d < k ? (rr * k + d) * 2u : OOB);
+            }
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+            for (int u = 0; u < SPB; u++) st[r * RS + u * LB_SLAB + lane] = e[r][u];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int u = 0; u < SPB; u++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) a[u][h] = *(const uint4 *)(st + c * RS + u * LB_SLAB + 16 * gq + 8 * h);
     }
     uint32_t mx = 0;
 #pragma unroll
@@ -452,13 +480,18 @@ hipError_t launch_lowbit_gemm(const WDev &w, size_t m, uint16_t *dst, const uint
     const uint32_t nslab = g.nsteps * 4;
     int8_t *q = (int8_t *)scratch;
     float *sp = (float *)((uint8_t *)scratch + lg_q_bytes(w, m));
-#define SMG_LG(SPB)                                                                                           \
-    hipLaunchKernelGGL(lowbit_quant_frag<SPB>, qgrid, dim3(256), 0, s, lhs, g.m, (uint32_t)w.k, nslab, g.mt16, \
-                       g.nbk, q, sp);                                                                         \
-    {                                                                                                         \
-        const hipError_t e = hipGetLastError();                                                               \
-        if (e != hipSuccess) return e;                                                                        \
-    }                                                                                                         \
+    const bool vec = (w.k & 7) == 0 && ((uintptr_t)lhs & 15) == 0;
+#define SMG_LG(SPB)                                                                                            \
+    if (vec)                                                                                                   \
+        hipLaunchKernelGGL((lowbit_quant_frag<SPB, true>), qgrid, dim3(256), 0, s, lhs, g.m, (uint32_t)w.k,    \
+                           nslab, g.mt16, g.nbk, q, sp);                                                       \
+    else                                                                                                       \
+        hipLaunchKernelGGL((lowbit_quant_frag<SPB, false>), qgrid, dim3(256), 0, s, lhs, g.m, (uint32_t)w.k,   \
+                           nslab, g.mt16, g.nbk, q, sp);                                                       \
+    {                                                                                                          \
+        const hipError_t e = hipGetLastError();                                                                \
+        if (e != hipSuccess) return e;                                                                         \
+    }                                                                                                          \
     return w.kind == W_Q2 ? launch_lg_rows<2, SPB>(g, ep, epv, s) : launch_lg_rows<1, SPB>(g, ep, epv, s);
     if (w.block == 64) { SMG_LG(1) }
     if (w.block == 128) { SMG_LG(2) }

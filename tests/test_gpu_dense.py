@@ -281,3 +281,41 @@ def test_odd_k_call_beside_another_threads_capture(smg):
         torch.cuda.synchronize()
         _check(d, want, k, False)
     _check(c, want, k, False)
+
+
+def test_odd_k_scratch_grows_beside_another_threads_capture(smg):
+    """As above with a smaller buffer there already: outgrown, it is given back
+    and replaced during the capture."""
+    import threading
+    import torch
+    m, n, k = 2000, 96, 1003
+    a, b = _mats(m, n, k, False, 71)
+    p = smg.prepack_f16(_bits(b), n, k)
+    other, cap = torch.cuda.Stream(), torch.cuda.Stream()
+    c, d = (torch.empty(m, n, dtype=torch.float16, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        smg.matmul_f16_packed(a[:16], p, c[:16], 16)
+    torch.cuda.synchronize()
+    err = []
+
+    def call():
+        try:
+            with torch.cuda.stream(other):
+                smg.matmul_f16_packed(a, p, c, m)
+        except Exception as e:  # noqa: BLE001
+            err.append(e)
+
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        smg.matmul_f16_packed(a, p, d, m)
+        t = threading.Thread(target=call)
+        t.start()
+        t.join()
+    assert not err, err
+    d.fill_(float("nan"))
+    g.replay()
+    torch.cuda.synchronize()
+    want = a.double() @ b.double()
+    _check(d, want, k, False)
+    _check(c, want, k, False)

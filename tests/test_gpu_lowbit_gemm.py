@@ -121,6 +121,24 @@ def test_many_rows_special_activations(smg, orc):
     assert np.array_equal(got[~nan(want)], want[~nan(want)])
 
 
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("m,n,k", [(70, 200, 512), (21, 130, 1001), (16, 64, 65)])
+def test_many_rows_of_an_unaligned_a(smg, orc, m, n, k, block):
+    """An A off 16-byte alignment, NaN around it: the rows' staged form, the same
+    bits as the oracle's."""
+    import torch
+    rng = np.random.default_rng(k + block)
+    a, codes, scales = _inputs(orc, rng, m, n, k, block, 2)
+    w = smg.Q2Weights(codes, scales, n, k, smg.Q2Params(block))
+    buf = torch.full((m * k + 16,), 0x7E00, dtype=torch.int16, device="cuda")
+    ad = buf[3:3 + m * k]
+    ad.copy_(torch.from_numpy(a.view(np.int16)))
+    c = torch.zeros(m * n, dtype=torch.int16, device="cuda")
+    smg.matmul_q2(ad, w, c, m)
+    want = orc.lowbit_reference(2, a, codes, scales, m, n, k, block)
+    assert np.array_equal(c.cpu().numpy().view(np.uint16), want)
+
+
 def test_noalloc_keeps_the_calls_it_took(smg, orc):
     """961 rows at K = 4096: the GEMM's scratch (16-row tiles) would pass the
     static array, the GEMV's fits it -- the call runs there, the same bits."""
