@@ -143,6 +143,72 @@ __device__ __forceinline__ float scale_mul_hi(uint32_t sc2, float s) {
     return r;
 }
 
+// Four cells' activation with the kind switch taken once, the f64 formulas as
+// act_f32 evaluates them.
+struct F4 {
+    float v[4];
+};
+__device__ __noinline__ F4 act4(uint32_t kind, F4 x, float alpha) {
+    const double a = (double)alpha;
+    switch (kind) {
+#define SMG_ACT4_CASE(K)                                                                                   \
+    case K:                                                                                                \
+        _Pragma("unroll") for (int e = 0; e < 4; e++) x.v[e] = (float)act_f64_body(K, (double)x.v[e], a);  \
+        break;
+        SMG_ACT4_CASE(1) SMG_ACT4_CASE(2) SMG_ACT4_CASE(3) SMG_ACT4_CASE(4) SMG_ACT4_CASE(5)
+        SMG_ACT4_CASE(6) SMG_ACT4_CASE(7) SMG_ACT4_CASE(8) SMG_ACT4_CASE(9) SMG_ACT4_CASE(10)
+        SMG_ACT4_CASE(11) SMG_ACT4_CASE(12) SMG_ACT4_CASE(13) SMG_ACT4_CASE(14)
+        SMG_ACT4_CASE(15) SMG_ACT4_CASE(16) SMG_ACT4_CASE(17) SMG_ACT4_CASE(18)
+        SMG_ACT4_CASE(19) SMG_ACT4_CASE(20) SMG_ACT4_CASE(21) SMG_ACT4_CASE(22)
+        SMG_ACT4_CASE(23) SMG_ACT4_CASE(24)
+#undef SMG_ACT4_CASE
+    default:
+        break;
+    }
+    return x;
+}
+
+// ep_cell for four cells side by side, each node's operands loaded together; a
+// cell past the output reads the last row's or column's.
+__device__ __forceinline__ void ep_cells4(const EpArgs &ep, float (&x)[4], const uint32_t (&row)[4],
+                                          const uint32_t (&col)[4], uint32_t m, uint32_t n, uint16_t (&h)[4]) {
+    for (uint32_t t = 0; t < ep.n_nodes; t++) {
+        const EpNode &nd = ep.nodes[t];
+        const uint16_t *p = (const uint16_t *)nd.ptr;
+        if (ep.fam[t] == EPF_ACT) {
+            if (t + 1 == ep.n_nodes && (nd.aux == 3 || nd.aux == 5)) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) h[j] = act_round16<false>(nd.aux, x[j], nd.scalar);
+                return;
+            }
+            F4 y;
+#pragma unroll
+            for (int j = 0; j < 4; j++) y.v[j] = x[j];
+            y = act4(nd.aux, y, nd.scalar);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = y.v[j];
+            continue;
+        }
+        uint16_t raw[4];
+        const uint32_t cls = ep.cls[t];
+        const size_t ld = nd.ld == 0 ? n : nd.ld;
+        if (cls == EPC_ROW || cls == EPC_COL || cls == EPC_TENSOR) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const size_t r = min(row[j], m - 1), c = min(col[j], n - 1);
+                raw[j] = p[cls == EPC_ROW ? r : cls == EPC_COL ? c : r * ld + c];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = ep_arith(ep.fam[t], x[j], f16_to_f32(raw[j]));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = ep_arith(ep.fam[t], x[j], nd.scalar);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) h[j] = f32_to_f16(x[j]);
+}
+
 // LDS bytes of a stage: row fragments, codes, scales and row scales (a block's
 // columns and rows each take one dword DMA of a wave, 256 bytes).
 template <int KIND, int SPB, int RT, int CT>
@@ -333,6 +399,28 @@ __global__ void __launch_bounds__(LG_NT, 2) lowbit_gemm(LgArgs g, EpArgs ep) {
             *(uint2 *)(stg + (i * 16 + c) * CS + wave * CT * 16 + ct * 16 + 4 * gq) = h;
         }
     __syncthreads();
+    if constexpr (EPV == 0) {
+        // four cells a thread, a row's columns side by side: the graph's steps are
+        // operand loads and f64 formulas in series, so the cells run side by side
+#pragma unroll 1
+        for (int i = t; i < RT * 16 * TN; i += 4 * LG_NT) {
+            float x[4];
+            uint32_t row[4], col[4];
+            uint16_t h[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int o = i + j * LG_NT;
+                row[j] = rt0 * 16 + o / TN;
+                col[j] = col0 + o % TN;
+                x[j] = f16_to_f32(stg[o / TN * CS + o % TN]);
+            }
+            ep_cells4(ep, x, row, col, g.m, g.n, h);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (row[j] < g.m && col[j] < g.n) g.dst[(size_t)row[j] * g.n + col[j]] = h[j];
+        }
+        return;
+    }
     const uint32_t cl = (t % (TN / 8)) * 8, col = col0 + cl;
     if (col >= g.n) return;  // no barrier follows
     const uint32_t ne = min(g.n - col, 8u);
@@ -350,20 +438,15 @@ __global__ void __launch_bounds__(LG_NT, 2) lowbit_gemm(LgArgs g, EpArgs ep) {
         if (row >= g.m) break;
         const uint4 c8 = *(const uint4 *)(stg + rl * CS + cl);
         uint32_t w4[4] = {c8.x, c8.y, c8.z, c8.w};
-        if constexpr (EPV != 1) {
+        if constexpr (EPV == 2) {
             uint32_t o4[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 if ((uint32_t)e >= ne) break;
                 float x = f16_to_f32((uint16_t)(w4[e / 2] >> (16 * (e % 2))));
-                uint16_t h;
-                if constexpr (EPV == 2) {
-                    if (g.col_a) x = x * va[e];
-                    x = x + vb[e];
-                    h = g.act == EP_ACT_NONE ? f32_to_f16(x) : act_round16<false>(g.act, x, g.act_alpha);
-                } else {
-                    h = ep_cell<false>(ep, x, row, col + e, g.n);
-                }
+                if (g.col_a) x = x * va[e];
+                x = x + vb[e];
+                const uint16_t h = g.act == EP_ACT_NONE ? f32_to_f16(x) : act_round16<false>(g.act, x, g.act_alpha);
                 o4[e / 2] |= (uint32_t)h << (16 * (e % 2));
             }
 #pragma unroll

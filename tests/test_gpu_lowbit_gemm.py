@@ -97,6 +97,50 @@ def test_wide_tiles_epilogue_bits(smg, orc, m, n, k, graph):
     assert np.array_equal(got, orc.matmul_lowbit_ep(2, a, codes, scales, m, n, k, block, nodes, act))
 
 
+@pytest.mark.parametrize("m,n", [(21, 77), (130, 8200)])
+def test_interpreted_store_every_node_bits(smg, orc, m, n):
+    """Graphs the stores are not compiled for: every activation last and, the
+    in-order ones, before another node; every operation with a scalar, row, column
+    and strided tensor operand. Ragged edges, one tile and many. (Where the
+    reference gives NaN, NaN.)"""
+    k, block, ld = 64, 64, n + 3
+    rng = np.random.default_rng(n)
+    a, codes, scales = _inputs(orc, rng, m, n, k, block, 2)
+    w = smg.Q2Weights(codes, scales, n, k, smg.Q2Params(block))
+    half = lambda lo, hi, size: orc.f32_to_f16(rng.uniform(lo, hi, size).astype(np.float32))  # noqa: E731
+    r, c, t = half(0.5, 1.5, m), half(-2, 2, n), half(0.5, 2, (m - 1) * ld + n)
+    plain = np.zeros(m * n, np.uint16)
+    smg.matmul_q2(a, w, plain, m)
+    few = m * n > 100000  # the oracle's time
+    graphs = []
+    for name, kind in smg.EP_ACT.items():
+        alpha = 0.3 if name in ("leaky_relu", "elu") else 0.0
+        arg = (0.3,) if alpha else ()
+        if few and kind not in (2, 3, 18):
+            continue
+        if kind <= 5:
+            graphs.append((getattr(smg.Epilogue().add_scalar(0.25), name)(), [(0, 0, 0.25, None, 0)], kind))
+            continue
+        node = (8, kind, float(np.float32(alpha)), None, 0)
+        graphs.append((getattr(smg.Epilogue().mul_row(r), name)(*arg), [(3, 0, 0.0, r, 0), node], None))
+        graphs.append((getattr(smg.Epilogue(), name)(*arg).mul_row(r), [node, (3, 0, 0.0, r, 0)], None))
+    for op in ("add", "sub", "mul", "div", "max", "min"):
+        g, nodes = smg.Epilogue(), []
+        for kind, v, s in (("scalar", None, 0.75), ("row", r, 0.0), ("col", c, 0.0), ("tensor", t, 0.0)):
+            f = g.max if (op, kind) == ("max", "scalar") else g.min if (op, kind) == ("min", "scalar") else getattr(
+                g, f"{op}_{kind}")
+            g = f(s) if v is None else f(v, ld=ld) if kind == "tensor" else f(v)
+            nodes.append((smg.EP_OP[f"{op}_{kind}"], 0, s, v, ld if kind == "tensor" else 0))
+        graphs.append((g, nodes, None))
+    nan = lambda x: (x & 0x7FFF) > 0x7C00  # noqa: E731
+    for ep, nodes, act in graphs:
+        got = np.full(m * n, 0x4880, np.uint16)
+        smg.matmul_q2_ep(a, w, got, m, ep)
+        want = orc.apply_ep(plain, m, n, nodes, act)
+        assert np.array_equal(nan(got), nan(want)), nodes
+        assert np.array_equal(got[~nan(want)], want[~nan(want)]), (nodes, act)
+
+
 def test_many_rows_special_activations(smg, orc):
     """Blocks of zeros, infinities, NaN and the smallest subnormals, and rows
     that differ only in one block: amax, inv and s as quantize_row gives them
