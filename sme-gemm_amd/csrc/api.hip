@@ -1805,12 +1805,14 @@ int smg_lowbit_matmul_dev(size_t m, const smg_weights *w, uint16_t *dst, const u
         // are quantized once into a buffer of this stream's own; where the
         // GEMM's whole tiles of rows would have to grow it while the stream is
         // captured, or do not fit the device, the GEMV's rows if they do
-        const size_t less = lowbit_scratch_bytes(w->d, m, &ea, sb - 1);
         scratch = dev_pool().find(w->device, stream, sb);
-        if (!scratch && less < sb && stream_capturing(stream) && (scratch = dev_pool().find(w->device, stream, less)))
-            sb = less;
-        if (!scratch) scratch = dev_pool().get(w->device, stream, sb);
-        if (!scratch && less < sb && (scratch = dev_pool().get(w->device, stream, less))) sb = less;
+        if (!scratch) {
+            const size_t less = lowbit_scratch_bytes(w->d, m, &ea, sb - 1);
+            if (less < sb && stream_capturing(stream)) scratch = dev_pool().find(w->device, stream, less);
+            if (scratch) sb = less;
+            else scratch = dev_pool().get(w->device, stream, sb);
+            if (!scratch && less < sb && (scratch = dev_pool().get(w->device, stream, less))) sb = less;
+        }
         if (!scratch) return fail(SMG_ENOMEM, "smg_lowbit_matmul_dev: scratch hipMalloc");
     }
     hipError_t e = launch_lowbit_gemv(w->d, m, dst, lhs, ea, scratch, sb, (hipStream_t)stream);
