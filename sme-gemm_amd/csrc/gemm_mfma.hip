@@ -521,7 +521,7 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
     if (read_dst && w.kind != W_F16 && w.kind != W_BF16) return hipErrorInvalidValue;
     if (!read_dst && q4r_supported(w, m, lhs_cs, lhs_rs, lhs, bf16))
         return launch_q4r(w, m, dst, dst_cs, dst_rs, lhs, lhs_rs, beta, ep, nullptr, 0, bf16, s);
-    if (!read_dst && gemm_mopa_supported(w, m, lhs_cs, lhs_rs, lhs))
+    if (!read_dst && gemm_mopa_supported(w, m, lhs_cs, lhs_rs, lhs) && gemm_mopa_pays(w, m, ep))
         return launch_gemm_mopa(w, m, dst, dst_cs, dst_rs, lhs, lhs_rs, beta, ep, s);
     if (w.kind == W_F16 || w.kind == W_BF16) {
         const DenseGemm d = {lhs, w.dense, dst, m, w.n, w.k, w.n_pad, lhs_rs, (long)w.k_pad, dst_rs, dst_cs,

@@ -334,6 +334,30 @@ bool gemm_mopa_supported(const WDev &w, size_t m, long lhs_cs, long lhs_rs, cons
            ((m + 127) / 128) * ((w.n + MP - 1) / MP) < big && mopa_tile(w, m) != 0;
 }
 
+// Whether the call's store leaves the product's gain. A tile stores 256 columns on
+// one compute unit where gemm_kernel's 128-column tiles use two, so a store that
+// takes long -- an interpreted graph with tensors or many nodes, an activation on
+// libm's exponentials -- needs more depth or a grid that fills the device.
+// gemm_kernel -> this (us), 1-bit: 129 x 128 x 512 with a tensor 22.6 -> 25.5, with
+// mish 36 -> 51, but with a row product 18.6 -> 17.8; 200 x 1000 x 1024 34.4 -> 36.6,
+// 54 -> 60, 29.0 -> 26.4, x 2048 50.2 -> 51.8, 70 -> 76; 300 x 4096 x 2048 52.7 ->
+// 52.6, 80 -> 76; 600 x 9000 x 1024 (180 tiles) 41.9 -> 40.1, 67 -> 63. 2-bit (256-row
+// tiles) 2100 x 4096 x 512 48.1 -> 53.0, 82 -> 94, 39.1 -> 28.1, x 1024 66.3 -> 65.5,
+// 100 -> 108.
+bool gemm_mopa_pays(const WDev &w, size_t m, const EpArgs &ep) {
+    bool longer = false, exps = false;
+    if (pick_ep(ep).v == 0) longer = ep.n_nodes > 4;
+    for (uint32_t i = 0; i < ep.n_nodes; i++) {
+        longer |= ep.cls[i] == EPC_TENSOR;
+        exps |= ep.fam[i] == EPF_ACT && ep.nodes[i].aux >= EP_ACT_EXP;
+    }
+    if (!longer && !exps) return true;
+    const size_t tiles = ((m + 127) / 128) * ((w.n + MP - 1) / MP);
+    if (w.k >= 4096 || (w.k >= 2048 && tiles >= 32)) return true;
+    if (tiles * 2 < (size_t)device_cus()) return false;
+    return exps ? mopa_tile(w, m) == 128 : w.k >= 1024;
+}
+
 hipError_t launch_gemm_mopa(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
                             long lhs_rs, float beta, const EpArgs &ep, hipStream_t s) {
     MopaArgs g = {};

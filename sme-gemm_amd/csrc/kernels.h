@@ -124,7 +124,8 @@ TileDims gemm_dense_tile_dims(size_t m, size_t n, size_t k);
 hipError_t launch_gemm_dense(const DenseGemm &d, const EpArgs &ep, bool bf16, hipStream_t s);
 
 // The f16 GEMM over low-bit weights (gemm_mopa.cuh); launch_gemm uses it
-// whenever gemm_mopa_supported holds.
+// whenever gemm_mopa_supported and gemm_mopa_pays hold.
+bool gemm_mopa_pays(const WDev &w, size_t m, const EpArgs &ep);
 bool gemm_mopa_supported(const WDev &w, size_t m, long lhs_cs, long lhs_rs, const uint16_t *lhs);
 TileDims gemm_mopa_tile(const WDev &w, size_t m);
 hipError_t launch_gemm_mopa(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,

@@ -2,6 +2,7 @@
 // code of the launch interface runs, nothing reaches a GPU.
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 
 #include "kernels.h"
 
@@ -107,6 +108,46 @@ int main(int argc, char **argv) {
                 CHECK(dense_pack_a_bytes(w, m, a + 1, 1, (long)k) != 0);         // unaligned rows
                 CHECK(dense_pack_a_bytes(w, m, a, (long)m, 1) != 0 || (m == 1 && k == 1));  // a column stride
             }
+    // Low-bit f16 products: what the tile serves, a long interpreted store aside.
+    {
+        const auto graph = [](std::initializer_list<uint32_t> ops, uint32_t act = 0) {
+            EpArgs ep = {};
+            for (uint32_t op : ops) {
+                ep.nodes[ep.n_nodes].op = op;
+                ep.nodes[ep.n_nodes].ptr = (const void *)256;
+                ep.fam[ep.n_nodes] = ep_family(op);
+                ep.cls[ep.n_nodes] = ep_class(op);
+                ep.n_nodes++;
+            }
+            if (act) {
+                ep.nodes[ep.n_nodes].op = EP_OP_ACT;
+                ep.nodes[ep.n_nodes].aux = act;
+                ep.fam[ep.n_nodes] = ep_family(EP_OP_ACT);
+                ep.cls[ep.n_nodes] = ep_class(EP_OP_ACT);
+                ep.n_nodes++;
+            }
+            return ep;
+        };
+        const EpArgs none = graph({}), bias = graph({EP_OP_ADD_COL}, EP_ACT_SILU), row = graph({EP_OP_MUL_ROW}),
+                     rtanh = graph({EP_OP_MUL_ROW}, EP_ACT_TANH), tensor = graph({EP_OP_ADD_COL, EP_OP_ADD_TENSOR}),
+                     five = graph({EP_OP_MUL_ROW, EP_OP_ADD_ROW, EP_OP_MUL_ROW, EP_OP_ADD_ROW, EP_OP_MUL_ROW}),
+                     mish = graph({EP_OP_MUL_ROW}, EP_ACT_MISH), bmish = graph({EP_OP_ADD_COL}, EP_ACT_MISH);
+        const struct {
+            int kind;
+            size_t m, n, k;
+            bool longer, exps;  // whether such graphs stay
+        } calls[] = {{W_Q1, 129, 128, 512, false, false},    {W_Q1, 200, 1000, 2048, false, false},
+                     {W_Q1, 200, 1000, 4096, true, true},    {W_Q1, 300, 4096, 2047, false, false},
+                     {W_Q1, 300, 4096, 2048, true, true},    {W_Q1, 600, 9000, 512, false, true},
+                     {W_Q1, 600, 9000, 1024, true, true},    {W_Q1, 2100, 4096, 512, false, false},
+                     {W_Q2, 2100, 4096, 1024, true, false},  {W_Q2, 2100, 4096, 2048, true, true}};
+        for (const auto &c : calls) {
+            const WDev w = lowbit(c.kind, c.n, c.k, 128);
+            for (const EpArgs *e : {&none, &bias, &row, &rtanh}) CHECK(gemm_mopa_pays(w, c.m, *e));
+            for (const EpArgs *e : {&tensor, &five}) CHECK(gemm_mopa_pays(w, c.m, *e) == c.longer);
+            for (const EpArgs *e : {&mish, &bmish}) CHECK(gemm_mopa_pays(w, c.m, *e) == c.exps);
+        }
+    }
     // Attention of row blocks: few short rows of a wide head stay on
     // attn_rows_mfma, as does what attn_rows_dma cannot address.
     {
