@@ -168,41 +168,50 @@ __device__ __noinline__ F4 act4(uint32_t kind, F4 x, float alpha) {
     return x;
 }
 
-// ep_cell for four cells side by side, each node's operands loaded together; a
-// cell past the output reads the last row's or column's.
-__device__ __forceinline__ void ep_cells4(const EpArgs &ep, float (&x)[4], const uint32_t (&row)[4],
-                                          const uint32_t (&col)[4], uint32_t m, uint32_t n, uint16_t (&h)[4]) {
+// Four cells' last activation, rounded: act_round16 four at a time.
+__device__ __forceinline__ void act_round4(uint32_t kind, const float (&x)[4], float alpha, uint16_t (&h)[4]) {
+    if (kind == EP_ACT_SILU || kind == EP_ACT_SIGMOID) {  // mostly without the f64 formula
+#pragma unroll
+        for (int j = 0; j < 4; j++) h[j] = act_round16<false>(kind, x[j], alpha);
+        return;
+    }
+    const F4 y = act4(kind, F4{{x[0], x[1], x[2], x[3]}}, alpha);
+#pragma unroll
+    for (int j = 0; j < 4; j++) h[j] = f32_to_f16(y.v[j]);
+}
+
+// ep_cell for four cells of a column side by side, each node's operands loaded
+// together; a row past the output reads the last one's.
+__device__ __forceinline__ void ep_cells4(const EpArgs &ep, float (&x)[4], const uint32_t (&row)[4], uint32_t col,
+                                          uint32_t m, uint32_t n, uint16_t (&h)[4]) {
     for (uint32_t t = 0; t < ep.n_nodes; t++) {
         const EpNode &nd = ep.nodes[t];
         const uint16_t *p = (const uint16_t *)nd.ptr;
         if (ep.fam[t] == EPF_ACT) {
-            if (t + 1 == ep.n_nodes && (nd.aux == 3 || nd.aux == 5)) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) h[j] = act_round16<false>(nd.aux, x[j], nd.scalar);
+            if (t + 1 == ep.n_nodes) {
+                act_round4(nd.aux, x, nd.scalar, h);
                 return;
             }
-            F4 y;
-#pragma unroll
-            for (int j = 0; j < 4; j++) y.v[j] = x[j];
-            y = act4(nd.aux, y, nd.scalar);
+            const F4 y = act4(nd.aux, F4{{x[0], x[1], x[2], x[3]}}, nd.scalar);
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = y.v[j];
             continue;
         }
-        uint16_t raw[4];
         const uint32_t cls = ep.cls[t];
         const size_t ld = nd.ld == 0 ? n : nd.ld;
-        if (cls == EPC_ROW || cls == EPC_COL || cls == EPC_TENSOR) {
+        if (cls == EPC_ROW || cls == EPC_TENSOR) {
+            uint16_t raw[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const size_t r = min(row[j], m - 1), c = min(col[j], n - 1);
-                raw[j] = p[cls == EPC_ROW ? r : cls == EPC_COL ? c : r * ld + c];
+                const size_t r = min(row[j], m - 1);
+                raw[j] = p[cls == EPC_ROW ? r : r * ld + col];
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = ep_arith(ep.fam[t], x[j], f16_to_f32(raw[j]));
         } else {
+            const float v = cls == EPC_COL ? f16_to_f32(p[col]) : nd.scalar;
 #pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = ep_arith(ep.fam[t], x[j], nd.scalar);
+            for (int j = 0; j < 4; j++) x[j] = ep_arith(ep.fam[t], x[j], v);
         }
     }
 #pragma unroll
@@ -386,7 +395,8 @@ __global__ void __launch_bounds__(LG_NT, 2) lowbit_gemm(LgArgs g, EpArgs ep) {
     wait_vm<0>();  // the steps issued past the last
 
     // Store: the f16 sums staged row-major in LDS (lane: 4 consecutive columns
-    // of its row), then each thread takes groups of 8 columns of a row.
+    // of its row), then each thread takes groups of 8 columns of a row, or, where
+    // the graph has an activation or is interpreted, four cells of a column.
     __syncthreads();
     uint16_t *stg = (uint16_t *)smem;
 #pragma unroll
@@ -399,25 +409,38 @@ __global__ void __launch_bounds__(LG_NT, 2) lowbit_gemm(LgArgs g, EpArgs ep) {
             *(uint2 *)(stg + (i * 16 + c) * CS + wave * CT * 16 + ct * 16 + 4 * gq) = h;
         }
     __syncthreads();
-    if constexpr (EPV == 0) {
-        // four cells a thread, a row's columns side by side: the graph's steps are
-        // operand loads and f64 formulas in series, so the cells run side by side
+    if (EPV == 0 || (EPV == 2 && g.act != EP_ACT_NONE)) {
+        // four cells of one column a thread: the graph's operand loads and the
+        // f64 formulas are chains, so the cells run side by side
+        static_assert(LG_NT % TN == 0, "a thread's column");
+        constexpr int RS = LG_NT / TN;  // rows a pass
+        const uint32_t cl = t % TN, col = col0 + cl;
+        if (col >= g.n) return;  // no barrier follows
+        const float va = EPV == 2 && g.col_a ? f16_to_f32(g.col_a[col]) : 1.0f;
+        const float vb = EPV == 2 ? f16_to_f32(g.col_b[col]) : 0.0f;
 #pragma unroll 1
-        for (int i = t; i < RT * 16 * TN; i += 4 * LG_NT) {
+        for (int rl = t / TN; rl < RT * 16; rl += 4 * RS) {
             float x[4];
-            uint32_t row[4], col[4];
+            uint32_t row[4];
             uint16_t h[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int o = i + j * LG_NT;
-                row[j] = rt0 * 16 + o / TN;
-                col[j] = col0 + o % TN;
-                x[j] = f16_to_f32(stg[o / TN * CS + o % TN]);
+                row[j] = rt0 * 16 + rl + j * RS;
+                x[j] = f16_to_f32(stg[(rl + j * RS) * CS + cl]);
             }
-            ep_cells4(ep, x, row, col, g.m, g.n, h);
+            if constexpr (EPV == 2) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (g.col_a) x[j] = x[j] * va;
+                    x[j] = x[j] + vb;
+                }
+                act_round4(g.act, x, g.act_alpha, h);
+            } else {
+                ep_cells4(ep, x, row, col, g.m, g.n, h);
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (row[j] < g.m && col[j] < g.n) g.dst[(size_t)row[j] * g.n + col[j]] = h[j];
+                if (row[j] < g.m) g.dst[(size_t)row[j] * g.n + col] = h[j];
         }
         return;
     }
@@ -445,9 +468,7 @@ __global__ void __launch_bounds__(LG_NT, 2) lowbit_gemm(LgArgs g, EpArgs ep) {
                 if ((uint32_t)e >= ne) break;
                 float x = f16_to_f32((uint16_t)(w4[e / 2] >> (16 * (e % 2))));
                 if (g.col_a) x = x * va[e];
-                x = x + vb[e];
-                const uint16_t h = g.act == EP_ACT_NONE ? f32_to_f16(x) : act_round16<false>(g.act, x, g.act_alpha);
-                o4[e / 2] |= (uint32_t)h << (16 * (e % 2));
+                o4[e / 2] |= (uint32_t)f32_to_f16(x + vb[e]) << (16 * (e % 2));
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) w4[e] = o4[e];
