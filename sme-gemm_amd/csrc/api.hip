@@ -1703,7 +1703,7 @@ int smg_gemm_run_dev(int bf16, size_t m, size_t n, size_t k, uint16_t *dst, long
     // B packed, and A where gemm_dense cannot read it (left where it is if only
     // B's share can be had)
     const size_t bb = round_up(d.n_pad * d.k_pad * 2, 256);
-    size_t ab = dense_pack_a_bytes(d, m, lhs, lhs_cs, lhs_rs);
+    size_t ab = strided_pack_a_bytes(d, m, lhs, lhs_cs, lhs_rs);
     if (ab && stream_capturing(stream) && !dev_pool().find(device, stream, bb + ab)) ab = 0;
     uint16_t *dense = (uint16_t *)dev_pool().get(device, stream, bb + ab);
     if (!dense && ab) {

@@ -589,6 +589,15 @@ size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs
         return 0;
     return rows * w.k_pad * 2;
 }
+// With B packed in the call as well, A's packing is a third launch, which few
+// short rows do not earn back: the call with A read and with A packed, us, 16 x
+// 500 x 63 14.6 / 15.5, 4 x 28 x 127 14.2 / 15.4, 200 x 64 x 63 15.1 / 15.6; the
+// other side of the lines: 61 x 499 x 63 16.3 / 15.5, 200 x 64 x 127 17.4 / 15.7,
+// 16 x 500 x 200 17.8 / 15.7.
+size_t strided_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs) {
+    const size_t ab = dense_pack_a_bytes(w, m, lhs, lhs_cs, lhs_rs);
+    return (m <= 32 ? w.k <= 128 : w.k <= 64 && m * w.n <= 16384) ? 0 : ab;
+}
 hipError_t launch_gemm_pack_a(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
                               long lhs_cs, long lhs_rs, float beta, const EpArgs &ep, bool bf16, uint16_t *scratch,
                               hipStream_t s, bool read_dst, float alpha) {

@@ -99,6 +99,8 @@ hipError_t launch_gemm(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long
 // (dense_pack_a_bytes, 16-byte aligned; 0 where launch_gemm reads A as well as
 // it is).
 size_t dense_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs);
+// The same where B is packed in the call too.
+size_t strided_pack_a_bytes(const WDev &w, size_t m, const uint16_t *lhs, long lhs_cs, long lhs_rs);
 hipError_t launch_gemm_pack_a(const WDev &w, size_t m, uint16_t *dst, long dst_cs, long dst_rs, const uint16_t *lhs,
                               long lhs_cs, long lhs_rs, float beta, const EpArgs &ep, bool bf16, uint16_t *scratch,
                               hipStream_t s, bool read_dst = false, float alpha = 0.0f);

@@ -108,6 +108,23 @@ int main(int argc, char **argv) {
                 CHECK(dense_pack_a_bytes(w, m, a + 1, 1, (long)k) != 0);         // unaligned rows
                 CHECK(dense_pack_a_bytes(w, m, a, (long)m, 1) != 0 || (m == 1 && k == 1));  // a column stride
             }
+    // A strided call packs A too, but for few short rows.
+    {
+        const size_t calls[][4] = {{32, 300, 127, 0}, {32, 300, 129, 1}, {33, 300, 63, 0},  {33, 300, 65, 1},
+                                   {200, 64, 63, 0},  {61, 499, 63, 1},  {1, 100, 8, 0},    {16, 500, 200, 1},
+                                   {128, 128, 63, 0}, {129, 128, 63, 1}, {3000, 500, 3001, 1}};
+        for (const auto &c : calls) {
+            WDev w = {};
+            w.kind = W_F16;
+            w.n = c[1];
+            w.k = c[2];
+            w.n_pad = (c[1] + 127) / 128 * 128;
+            w.k_pad = (c[2] + 63) / 64 * 64;
+            w.dense = (const uint16_t *)4096;
+            const uint16_t *a = (const uint16_t *)256;
+            CHECK((strided_pack_a_bytes(w, c[0], a, (long)c[0], 1) != 0) == (c[3] != 0));
+        }
+    }
     // Low-bit f16 products: what the tile serves, a long interpreted store aside.
     {
         const auto graph = [](std::initializer_list<uint32_t> ops, uint32_t act = 0) {

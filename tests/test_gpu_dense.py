@@ -146,6 +146,24 @@ def test_products_over_any_k(smg, m, n, k, bf16):
     _check(c, want + 0.5 * c0.double(), k, bf16)
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("m,n,k", [(32, 300, 127), (32, 300, 129), (33, 300, 63), (33, 300, 65), (128, 128, 63),
+                                   (129, 128, 63), (1, 1, 1)])
+def test_strided_calls_with_and_without_a_packed(smg, m, n, k, bf16):
+    """Both sides of the line up to which a strided call reads such an A where
+    it is: the packed weights' call, which always packs it, gives the same
+    bits."""
+    import torch
+    a, b = _mats(m, n, k, bf16, m + k)
+    p = (smg.prepack_bf16 if bf16 else smg.prepack_f16)(_bits(b), n, k)
+    c, e = (torch.empty(m, n, dtype=a.dtype, device="cuda") for _ in range(2))
+    (smg.matmul_bf16_packed if bf16 else smg.matmul_f16_packed)(a, p, e, m)
+    at = a.t().contiguous()
+    (smg.gemm_bf16 if bf16 else smg.gemm_f16)(m, n, k, c, n, 1, at, 1, m, b, n, 1, 0.0, 1.0)
+    _check(c, a.double() @ b.double(), k, bf16)
+    assert torch.equal(c.view(torch.int16), e.view(torch.int16))
+
+
 def test_odd_k_product_captured_without_scratch(smg):
     """A first odd-K product on a stream under capture allocates nothing (it
     reads A as it is) and replays right; eager calls on the stream then pack."""
